@@ -35,7 +35,7 @@ hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 // the retired buffers of a slot add up to at most twice its final size.  Not
 // safe for concurrent calls from several threads (the reference's scratch has
 // the same property, src/k_gemv.hip:47-51).
-enum Slot { kSlotActQ = 0, kSlotActS = 1, kSlotGemmA = 2, kSlotGemmPart = 3, kSlotGemmCnt = 4, kSlotAttnPart = 5, kSlotGemvPart = 6, kSlotGemvCnt = 7, kSlotAttnCnt = 8, kSlotAttnKV = 9, kSlots = 10 };
+enum Slot { kSlotActQ = 0, kSlotActS = 1, kSlotGemmA = 2, kSlotGemmPart = 3, kSlotAttnPart = 4, kSlotGemvPart = 5, kSlotGemvCnt = 6, kSlotAttnCnt = 7, kSlotAttnKV = 8, kSlots = 9 };
 constexpr int kMaxDev = 64;
 struct Buf {
     void* p = nullptr;
@@ -157,12 +157,10 @@ int run_gemm(const char* who, int32_t* gsum, float* c, const uint32_t* wq, const
     int cus = 0, rc = device_cus(&cus);
     if (rc) return rc;
     const rt4::GemmPlan plan = rt4::gemm_plan(M, N, K, cus);
-    void *part = nullptr, *cnt = nullptr;
+    void* part = nullptr;
     if ((rc = lib_scratch(kSlotGemmPart, plan.part_bytes, &part, st))) return rc;
-    if ((rc = lib_scratch(kSlotGemmCnt, plan.cnt_bytes, &cnt, st, true))) return rc;
-    return hip_status(rt4::launch_gemm_w4a8(c, gsum, xq, wq, sc, wsc_gm, M, N, K, plan, static_cast<float*>(part),
-                                            static_cast<int*>(cnt), st),
-                      who);
+    return hip_status(
+        rt4::launch_gemm_w4a8(c, gsum, xq, wq, sc, wsc_gm, M, N, K, plan, static_cast<float*>(part), st), who);
 }
 
 // The GEMV launch with its balanced grid: split tiles need a small partial

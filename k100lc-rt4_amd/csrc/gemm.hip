@@ -13,10 +13,10 @@
 // 16*I_h + I_l = I exactly, so here the digits are recombined into int8 once
 // and a single int8 contraction runs on v_mfma_i32_32x32x32_i8.
 //
-// Tiling.  Workgroup tile 128 activation rows x 256 weight rows, 8 waves; wave w
-// owns weight rows (output columns) 32w..32w+31 and all 128 activation rows, i.e.
-// four 32 x 32 row tiles sharing one weight fragment, so each wave unpacks only
-// its own 32 weight rows.  One 128-wide K group ("unit" = one tile x one group)
+// Tiling.  Workgroup tile 32 RT activation rows x 256 weight rows, 8 waves; wave w
+// owns weight rows (output columns) 32w..32w+31 and all the activation rows, i.e. RT
+// 32 x 32 row tiles (four, unless M is small) sharing one weight fragment, so each wave
+// unpacks only its own 32 weight rows.  One 128-wide K group ("unit" = one tile x one group)
 // is four MFMA k-steps per row tile.  The int32 accumulators restart at every
 // group and are folded into fp32:
 //     facc += f32(acc) * S,   S = sa * sb,   acc = 16*I exactly (x16 nibble unpack),
@@ -59,14 +59,23 @@
 // 16 consecutive fragment rows of a ds_read_b128 hit 16 distinct 16-byte bank
 // groups.
 //
-// Scheduling ("stream-K").  One persistent workgroup per CU takes an equal,
-// contiguous share of the (tile, group) units, numbered so each XCD owns a
-// contiguous slice.  A tile split between workgroups is combined
-// deterministically: every contributor except the last writes its fp32 partial
-// to a workspace slot (agent-coherent stores), bumps the tile's counter, and the
-// contributor that arrives last sums all partials in workgroup order and writes
-// C; it also resets the counter for the next call.  No workgroup ever waits for
-// another.
+// Scheduling.  One persistent workgroup per CU.  With `rem` the tile count modulo the
+// workgroup count, the first rem tiles are shared out by (tile, group) units, an equal
+// contiguous range each; every workgroup then takes the same number of whole tiles.
+// Whole tiles need no partial sums: at M=1024, N=17408, K=5120 (544 tiles) two of the
+// three segments of a workgroup are whole, where equal ranges over all units ("stream-K"
+// throughout) made two of three split: 64 MB of partials written and read back became 32
+// (144 -> 127 us with the combining below; M=2048 262 -> 249).  A part of a tile goes to
+// a workspace slot and gemm_combine_k sums the parts in workgroup order, so results do
+// not depend on timing and no workgroup waits for another.  Workgroups of one XCD take
+// neighbouring tiles (the same weights).
+//
+// Row tiles.  RT = 4 (128 rows) from 65 rows up; RT = 2 and 1 for up to 64 and 32 rows,
+// whose units issue less (a unit of RT = 4 takes ~1.36 us here, RT = 2 0.87, RT = 1 0.60:
+// the weight unpack, the barrier and the bookkeeping stay) and whose partials are half
+// and a quarter of the size.  N=17408 K=5120, GEMM and combining launch, us: M=37 33.7 ->
+// 16.2 + 4.9, of which the weights' one-pass read alone is 8.4; the 128-row form computed
+// all 128 rows for any M.
 #include "rt4_dev.h"
 #include "rt4_internal.h"
 
@@ -74,84 +83,64 @@ namespace rt4 {
 namespace {
 
 typedef __attribute__((address_space(3))) void lds_void;
-typedef float v4f __attribute__((ext_vector_type(4)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef float v32f __attribute__((ext_vector_type(32)));
 
-constexpr int BM = 128;           // activation rows per tile
 constexpr int BN = 256;           // weight rows (output columns) per tile
 constexpr int NT = 512;           // 8 waves
 constexpr int NS = 4;             // LDS stages
-constexpr int A_ST = BM * 128;    // int8 activation tile per stage
 constexpr int B_ST = BN * 64;     // packed weight tile per stage
 constexpr int S_ST = 2048;        // sa (512 B) + sb (1024 B) + 512 B written by the two idle waves
-constexpr int LDS_B = 0;                       // weight stages
-constexpr int LDS_A = LDS_B + NS * B_ST;       // activation stages
-constexpr int LDS_S = LDS_A + NS * A_ST;       // scale stages
-constexpr int LDS_FLAG = LDS_S + NS * S_ST;
-constexpr int LDS_META = LDS_FLAG + 16;            // split-tile metadata (10 ints)
-constexpr int LDS_BYTES = LDS_META + 48;
-constexpr int DMA_PER_UNIT = 5;   // DMA instructions per wave per unit
-constexpr int PART_FLOATS = NT * 64;   // one partial tile: 64 outputs per thread, [k][thread]
 
-// Device-scope (sc1) 16-byte stores / loads of split-tile partials, the cache
-// policy of agent-scope atomics: the stores write through the per-XCD L2 and
-// are in memory once the writer's s_waitcnt has retired them, and the loads
-// read the coherent copy.  Four at a time (one row tile's 16 values per lane,
-// at a stride of NT*4 floats), each with its wait in the same asm statement:
-// store data registers must not be overwritten before the stores have read them,
-// and loaded registers must not be touched before they are valid, neither of
-// which the compiler can know for asm memory operations.
-__device__ __forceinline__ void store4_dev16(float* p, const v16i& f) {
-    constexpr size_t S = (size_t)NT * 4;
-    const v4i v0 = __builtin_shufflevector(f, f, 0, 1, 2, 3), v1 = __builtin_shufflevector(f, f, 4, 5, 6, 7);
-    const v4i v2 = __builtin_shufflevector(f, f, 8, 9, 10, 11), v3 = __builtin_shufflevector(f, f, 12, 13, 14, 15);
-    asm volatile(
-        "global_store_dwordx4 %0, %4, off sc1\n\t"
-        "global_store_dwordx4 %1, %5, off sc1\n\t"
-        "global_store_dwordx4 %2, %6, off sc1\n\t"
-        "global_store_dwordx4 %3, %7, off sc1\n\t"
-        "s_waitcnt vmcnt(0) expcnt(0)"
-        :
-        : "v"(p), "v"(p + S), "v"(p + 2 * S), "v"(p + 3 * S), "v"(v0), "v"(v1), "v"(v2), "v"(v3)
-        : "memory");
-}
-__device__ __forceinline__ void add4_dev16(v16i& f, const float* p) {
-    constexpr size_t S = (size_t)NT * 4;
-    v4f v0, v1, v2, v3;
-    asm volatile(
-        "global_load_dwordx4 %0, %4, off sc1\n\t"
-        "global_load_dwordx4 %1, %5, off sc1\n\t"
-        "global_load_dwordx4 %2, %6, off sc1\n\t"
-        "global_load_dwordx4 %3, %7, off sc1\n\t"
-        "s_waitcnt vmcnt(0)"
-        : "=&v"(v0), "=&v"(v1), "=&v"(v2), "=&v"(v3)
-        : "v"(p), "v"(p + S), "v"(p + 2 * S), "v"(p + 3 * S)
-        : "memory");
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        f[e] = __float_as_int(__int_as_float(f[e]) + v0[e]);
-        f[4 + e] = __float_as_int(__int_as_float(f[4 + e]) + v1[e]);
-        f[8 + e] = __float_as_int(__int_as_float(f[8 + e]) + v2[e]);
-        f[12 + e] = __float_as_int(__int_as_float(f[12 + e]) + v3[e]);
-    }
+// Sizes that depend on the row tiles per workgroup tile, RT = 1, 2 or 4 (32, 64 or 128
+// activation rows).
+template <int RT>
+struct Tile {
+    static constexpr int BM = 32 * RT;
+    static constexpr int A_DMA = RT == 4 ? 2 : 1;         // activation DMA instructions per wave (8 rows each)
+    static constexpr int A_ST = A_DMA * 8 * 1024;         // int8 activation rows per stage (64 for RT = 1 too:
+                                                          // rows 32.. are loaded and not read)
+    static constexpr int LDS_B = 0;                       // weight stages
+    static constexpr int LDS_A = LDS_B + NS * B_ST;       // activation stages
+    static constexpr int LDS_S = LDS_A + NS * A_ST;       // scale stages
+    static constexpr int LDS_BYTES = LDS_S + NS * S_ST;
+    static constexpr int DMA_PER_UNIT = A_DMA + 3;        // DMA instructions per wave per unit
+    static constexpr int PART_FLOATS = NT * 16 * RT;      // one partial tile: 16 RT outputs per thread, [k][thread]
+};
+
+// Split-tile partials go through buffer stores and loads with the device-scope cache
+// policy (sc1, that of agent-scope atomics): the stores write through the per-XCD L2
+// and are in memory once the writer's s_waitcnt has retired them, and the loads read
+// the coherent copy.  All 16 of a thread's stores, and all 16 loads of one
+// contributor's partial, are in flight together: one round trip each where four
+// 16-byte groups with a wait of their own took four.
+constexpr int kSc1 = 16;               // cache policy: sc1
+constexpr int kRsrcW3 = 0x00020000;    // dword 3 of a buffer resource: 32-bit data format
+template <int RT>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t part_rsrc(float* part, int slot) {
+    return __builtin_amdgcn_make_buffer_rsrc(part + (size_t)slot * Tile<RT>::PART_FLOATS, 0,
+                                             Tile<RT>::PART_FLOATS * (int)sizeof(float), kRsrcW3);
 }
 
 // Per-lane byte offsets of this wave's DMA sources for one tile (relative to the
 // unit's scalar bases), unchanged while the tile is.  LDS layouts:
-//   A  [128 rows][8 x 16 B], 16-byte chunk c of row r stored at c ^ ((r >> 1) & 7);
-//      wave w loads rows 16w..16w+15 (two instructions of 8 rows x 128 B)
+//   A  [rows][8 x 16 B], 16-byte chunk c of row r stored at c ^ ((r >> 1) & 7); wave w
+//      loads rows 8w.. (RT = 4: 16w.., two instructions), 8 rows x 128 B each
 //   B  [256 rows][4 x 16 B] packed, chunk c of row r stored at c ^ ((r >> 2) & 3);
 //      wave w loads rows 32w..32w+31, the ones it reads
 //   S  sa[128] f32 (waves 0, 1), sb[256] f32 (waves 2..5); waves 6, 7 repeat an sb
 //      load into the spare 512 B so that every wave issues the same count.
+template <int RT>
 struct DmaOff {
-    uint32_t a[2], b[2], s;
+    uint32_t a[Tile<RT>::A_DMA], b[2], s;
 };
-__device__ __forceinline__ DmaOff dma_offsets(int bm, int bn, int M, int N, int K, int w, int lane) {
-    DmaOff o;
+template <int RT>
+__device__ __forceinline__ DmaOff<RT> dma_offsets(int bm, int bn, int M, int N, int K, int w, int lane) {
+    constexpr int A_DMA = Tile<RT>::A_DMA;
+    DmaOff<RT> o;
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-        const int r = 16 * w + 8 * t + (lane >> 3);
+    for (int t = 0; t < A_DMA; t++) {
+        const int r = 8 * (A_DMA * w + t) + (lane >> 3);
         const int c = (lane & 7) ^ ((r >> 1) & 7);
         const int gr = min(bm + r, M - 1);
         o.a[t] = (uint32_t)gr * (uint32_t)K + c * 16;
@@ -170,9 +159,18 @@ __device__ __forceinline__ DmaOff dma_offsets(int bm, int bn, int M, int N, int 
     return o;
 }
 
-// Which workgroup's share contains unit u (shares are [T*b/P, T*(b+1)/P)).
-__device__ __forceinline__ int owner_of(long long u, long long T, int P) {
-    return (int)(((u + 1) * P - 1) / T);
+// First unit of range b: floor(R b / Pr) with R = q Pr + r, in 32 bits (rem < 2^16 tiles,
+// r and b < Pr <= the CU count).
+__device__ __forceinline__ int range_start(const GemmSched& s, int b) {
+    return s.q * b + (int)((unsigned)(s.r * b) / (unsigned)s.Pr);
+}
+// The range that holds unit u: an estimate, corrected to range_start(b) <= u < range_start(b + 1).
+__device__ __forceinline__ int owner_of(const GemmSched& s, int u) {
+    int b = (int)((float)u / ((float)s.q + (float)s.r / (float)s.Pr));
+    b = min(max(b, 0), s.Pr - 1);
+    while (range_start(s, b) > u) b--;
+    while (range_start(s, b + 1) <= u) b++;
+    return b;
 }
 
 // Tile coordinates of a unit, as the flush and the group-sum stores need them.
@@ -180,27 +178,40 @@ struct TileRef {
     int t, bm, bn, g;
 };
 
-template <bool GSUM>
+template <int RT, bool GSUM>
 __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ A,
                                                      const uint32_t* __restrict__ W,
                                                      const float* __restrict__ sa,
                                                      const float* __restrict__ sb,
                                                      float* __restrict__ C,
                                                      int32_t* __restrict__ gsum,
-                                                     float* __restrict__ part,
-                                                     int* __restrict__ cnt, int M, int N, int K,
-                                                     int ntm, long long T) {
-    __shared__ __align__(16) unsigned char lds[LDS_BYTES];
-    int* s_flag = reinterpret_cast<int*>(lds + LDS_FLAG);
+                                                     float* __restrict__ part, int M, int N, int K,
+                                                     GemmSched sch) {
+    using TL = Tile<RT>;
+    constexpr int BM = TL::BM, A_ST = TL::A_ST, DMA_PER_UNIT = TL::DMA_PER_UNIT;
+    constexpr int LDS_A = TL::LDS_A, LDS_B = TL::LDS_B, LDS_S = TL::LDS_S;
+    __shared__ __align__(16) unsigned char lds[TL::LDS_BYTES];
     const int lane = threadIdx.x & 63;
     const int w = uniform(threadIdx.x >> 6);
     const int lr = lane & 31, lh = lane >> 5;
     const int NG = K >> 7;
     const int P = gridDim.x;
     const int b = (P % 8 == 0) ? (int)(blockIdx.x % 8) * (P / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
-    const long long u0 = T * b / P, u1 = T * (b + 1) / P;
-    const int n = (int)(u1 - u0);
-    const int first_tile = (int)(u0 / NG);
+    // This workgroup's work: its range [r0, r1) of the remainder tiles' units (the first
+    // sch.rem tiles, shared by the first sch.Pr workgroups), then sch.full whole tiles,
+    // P apart.  rl_t, rl_e: the last remainder tile of the range and the group it ends
+    // before (-1: no range).
+    const int ntm = sch.ntm;
+    const int r0 = b < sch.Pr ? range_start(sch, b) : 0, r1 = b < sch.Pr ? range_start(sch, b + 1) : 0;
+    const int n = r1 - r0 + sch.full * NG;
+    if (n == 0) return;
+    const int rl_t = r1 > r0 ? (r1 - 1) / NG : -1, rl_e = r1 > r0 ? r1 - rl_t * NG : 0;
+    const int t_first = r1 > r0 ? r0 / NG : sch.rem + b;
+    const int g_first = r1 > r0 ? r0 - t_first * NG : 0;
+    auto next_tile = [&](int t) __attribute__((always_inline)) -> int {
+        return t < rl_t ? t + 1 : t < sch.rem ? sch.rem + b : t + P;
+    };
+    auto seg_end = [&](int t) __attribute__((always_inline)) -> int { return t == rl_t ? rl_e : NG; };
 
     // per-lane LDS read offsets into the current stage (next_stage moves them on);
     // the row tile is an immediate
@@ -218,14 +229,14 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
     int rsa = LDS_S + lane * 4, rsb = LDS_S + 512 + (32 * w + lr) * 4;
     // per-wave LDS destinations of the DMA (m0 = base + stage immediate)
     const uint32_t L = lds_addr(lds);
-    const uint32_t dstA = L + LDS_A + 2 * w * 1024, dstB = L + LDS_B + 2 * w * 1024;
+    const uint32_t dstA = L + LDS_A + TL::A_DMA * w * 1024, dstB = L + LDS_B + 2 * w * 1024;
     const uint32_t dstS = L + LDS_S + (w < 2 ? w * 256 : w < 6 ? 512 + (w - 2) * 256 : 1536);
 
     // facc[ii]: row tile ii (rows 32 ii..32 ii+31) x this wave's 32 columns; lane (lr, lh)
     // holds column 32w + lr, rows 32 ii + 8q + 4lh + e in register 4q + e.
-    v16i facc[4];
+    v16i facc[RT];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < RT; i++)
 #pragma unroll
         for (int r = 0; r < 16; r++) facc[i][r] = 0;
 
@@ -268,97 +279,65 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
         }
     };
 
-    // End of this workgroup's segment of tile x.t: publish it (see the file comment).
-    // Split-tile metadata of this workgroup's first and last tile (only these can be
-    // shared with other workgroups), formed once here so that the flush, which runs
-    // amid the pipeline's live registers, needs no 64-bit arithmetic:
-    //   [0] first tile, [1] whole, [2] owner of its first unit, [3] owner of its last
-    //   unit, [4] partial slot of that first owner; [5..9] the same for the last tile.
-    // A contributor v writes its partial of tile t to slot 2v (t is v's first tile) or
-    // 2v + 1 (its last tile).  Every contributor after the first owner starts its
-    // share inside t, so t is its first tile; the first owner's slot is 0 only if its
-    // share starts exactly at the tile's first unit.
-    int* meta = reinterpret_cast<int*>(lds + LDS_META);
-    if (threadIdx.x == 0) {
-        const long long tl = (u1 - 1) / NG;
+    // C of the tile at (bm, bn) from f.  A wave whose columns all exist in a tile whose
+    // rows all exist stores with the row as a scalar offset (one vector instruction per
+    // value besides the store, where 64-bit addresses took four); edges go row by row
+    // with the buffer's range check dropping the rows past M, and drain their stores.
+    // (N passes through an empty asm: the row offsets are then formed here, in this
+    // rare path, instead of being hoisted out of the loops into registers.)
+    auto write_c = [&](const v16i (&f)[RT], int bm, int bn) __attribute__((always_inline)) {
+        uint32_t Nb = (uint32_t)N * 4u;
+        asm volatile("" : "+s"(Nb));
+        const uint32_t nn = (uint32_t)(bn + 32 * w + lr);
+        const int rows = min(M - bm, BM);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            reinterpret_cast<char*>(C) + (size_t)bm * Nb, 0, (int)((uint32_t)rows * Nb), kRsrcW3);
+        const uint32_t vo = (uint32_t)(4 * lh) * Nb + nn * 4u;
+        if (rows == BM && bn + 32 * w + 32 <= N) {
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const long long t = e ? tl : (long long)first_tile;
-            const long long tb = t * NG, te = tb + NG;
-            const int wf = owner_of(tb, T, P), wl = owner_of(te - 1, T, P);
-            meta[5 * e + 0] = (int)t;
-            meta[5 * e + 1] = (u0 <= tb && u1 >= te);
-            meta[5 * e + 2] = wf;
-            meta[5 * e + 3] = wl;
-            meta[5 * e + 4] = (T * wf / P == tb) ? 0 : 1;
-        }
-    }
-
-    // End of this workgroup's segment of tile x.t: publish it (see the file comment).
-    auto flush = [&](const TileRef& x) __attribute__((always_inline)) {
-        // only the first and the last tile of a share can be split; tiles between are whole
-        const int tf = uniform(meta[0]), tl = uniform(meta[5]);
-        const int e = x.t == tf ? 0 : 5;
-        const bool whole = (x.t != tf && x.t != tl) || uniform(meta[e + 1]);
-        bool write_c = true;
-        if (!whole) {
-            const int wf = uniform(meta[e + 2]), wl = uniform(meta[e + 3]), slot_f = uniform(meta[e + 4]);
-            float* my = part + ((size_t)b * 2 + (e ? 1 : 0)) * PART_FLOATS + (size_t)threadIdx.x * 4;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            for (int ii = 0; ii < RT; ii++)
 #pragma unroll
-            for (int ii = 0; ii < 4; ii++) store4_dev16(my + (size_t)ii * 4 * NT * 4, facc[ii]);
-            __syncthreads();
-            if (threadIdx.x == 0)
-                *s_flag = __hip_atomic_fetch_add(cnt + x.t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == wl - wf;
-            __syncthreads();
-            write_c = *s_flag;
-            if (write_c) {
-#pragma unroll
-                for (int ii = 0; ii < 4; ii++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) facc[ii][r] = 0;
-                for (int v = wf; v <= wl; v++) {
-                    const int slot = 2 * v + (v == wf ? slot_f : 0);
-                    const float* pp = part + (size_t)slot * PART_FLOATS + (size_t)threadIdx.x * 4;
-#pragma unroll
-                    for (int ii = 0; ii < 4; ii++) add4_dev16(facc[ii], pp + (size_t)ii * 4 * NT * 4);
+                for (int r = 0; r < 16; r++) {
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(__int_as_float(f[ii][r]) * 0.0625f), rs, vo,
+                                                          (32 * ii + 8 * (r >> 2) + (r & 3)) * Nb, 0);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                if (threadIdx.x == 0) __hip_atomic_store(cnt + x.t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        if (write_c) {
-            // N passes through an empty asm: the row offsets below are then formed here,
-            // in this rare path, instead of being hoisted out of the loops into registers
-            // held for the whole kernel.
-            int Nv = N;
-            asm volatile("" : "+s"(Nv));
-            const uint32_t nn = (uint32_t)(x.bn + 32 * w + lr);
-            float* cb = C + (size_t)x.bm * Nv + nn;
-            const int mrows = M - x.bm;
+        } else {
             if (nn < (uint32_t)N) {
-                if (mrows >= BM) {
 #pragma unroll
-                    for (int ii = 0; ii < 4; ii++)
-#pragma unroll
-                        for (int r = 0; r < 16; r++) {
-                            const int ml = 32 * ii + 8 * (r >> 2) + 4 * lh + (r & 3);
-                            cb[(size_t)ml * Nv] = __int_as_float(facc[ii][r]) * 0.0625f;
-                            __builtin_amdgcn_sched_barrier(0);   // one address at a time
-                        }
-                } else {
-#pragma unroll
-                    for (int ii = 0; ii < 4; ii++)
+                for (int ii = 0; ii < RT; ii++)
+                    if (32 * ii < rows) {
 #pragma unroll
                         for (int r = 0; r < 16; r++) {
-                            const int ml = 32 * ii + 8 * (r >> 2) + 4 * lh + (r & 3);
-                            if (ml < mrows) cb[(size_t)ml * Nv] = __int_as_float(facc[ii][r]) * 0.0625f;
+                            __builtin_amdgcn_raw_buffer_store_b32(
+                                __float_as_uint(__int_as_float(f[ii][r]) * 0.0625f), rs,
+                                vo + (32 * ii + 8 * (r >> 2) + (r & 3)) * Nb, 0, 0);
                             __builtin_amdgcn_sched_barrier(0);
                         }
-                }
+                    }
             }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+    };
+    // End of this workgroup's segment of tile x.t: a whole tile is written out; a part
+    // of one goes to its partial slot, 2b for this workgroup's first tile and 2b + 1 for
+    // its last remainder tile, for gemm_combine_k.  Nothing is waited for here.
+    auto flush = [&](const TileRef& x, bool whole) __attribute__((always_inline)) {
+        if (whole) {
+            write_c(facc, x.bm, x.bn);
+        } else {
+            const __amdgpu_buffer_rsrc_t rs = part_rsrc<RT>(part, 2 * b + (x.t == t_first ? 0 : 1));
+#pragma unroll
+            for (int ii = 0; ii < RT; ii++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    __builtin_amdgcn_raw_buffer_store_b128(
+                        v4u{(unsigned)facc[ii][4 * q], (unsigned)facc[ii][4 * q + 1], (unsigned)facc[ii][4 * q + 2],
+                            (unsigned)facc[ii][4 * q + 3]},
+                        rs, threadIdx.x * 16, (4 * ii + q) * NT * 16, kSc1);
         }
 #pragma unroll
-        for (int ii = 0; ii < 4; ii++)
+        for (int ii = 0; ii < RT; ii++)
 #pragma unroll
             for (int r = 0; r < 16; r++) facc[ii][r] = 0;
     };
@@ -366,38 +345,31 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
     // ---- DMA side: the unit being loaded.  Its sources are the kernel arguments
     // (scalar bases) plus per-lane 32-bit offsets that hold the row, the chunk and
     // the group: each unit adds one group to them, a new tile recomputes them.
-    int dleft, dtm, dtn, dg0;
-    {
-        const int t0 = (int)(u0 / NG);
-        dg0 = (int)(u0 - (long long)t0 * NG);
-        dleft = NG - dg0;
-        dtn = t0 / ntm;
-        dtm = t0 - dtn * ntm;
-    }
+    int dt = t_first, dleft = seg_end(t_first) - g_first;
+    int dtn = dt / ntm, dtm = dt - dtn * ntm;
     const void* sbase = (w < 2 ? (const void*)sa : (const void*)sb);
     const uint32_t s_step = (w < 2 ? (uint32_t)M : (uint32_t)N) * 4u;
-    DmaOff off = dma_offsets(dtm * BM, dtn * BN, M, N, K, w, lane);
+    DmaOff<RT> off = dma_offsets<RT>(dtm * BM, dtn * BN, M, N, K, w, lane);
     // the group moves the (scalar) source bases; the per-lane offsets change per tile
-    const char* bA = reinterpret_cast<const char*>(A) + (size_t)dg0 * 128;
-    const char* bW = reinterpret_cast<const char*>(W) + (size_t)dg0 * 64;
-    const char* bS = reinterpret_cast<const char*>(sbase) + (size_t)dg0 * s_step;
+    const char* bA = reinterpret_cast<const char*>(A) + (size_t)g_first * 128;
+    const char* bW = reinterpret_cast<const char*>(W) + (size_t)g_first * 64;
+    const char* bS = reinterpret_cast<const char*>(sbase) + (size_t)g_first * s_step;
     // DMA of the unit at the DMA side's position into stage st
     auto issue = [&](int st) __attribute__((always_inline)) {
         const uint32_t da = dstA + st * A_ST, db = dstB + st * B_ST, ds = dstS + st * S_ST;
         dma16<0>(off.a[0], bA, da);
-        dma16<1024>(off.a[1], bA, da);
+        if constexpr (TL::A_DMA == 2) dma16<1024>(off.a[1], bA, da);
         dma16<0>(off.b[0], bW, db);
         dma16<1024>(off.b[1], bW, db);
         dma4<0>(off.s, bS, ds);
     };
     auto advance_dma = [&]() __attribute__((always_inline)) {
         if (--dleft == 0) {
-            dleft = NG;
-            if (++dtm == ntm) {
-                dtm = 0;
-                ++dtn;
-            }
-            off = dma_offsets(dtm * BM, dtn * BN, M, N, K, w, lane);
+            dt = next_tile(dt);
+            dleft = seg_end(dt);
+            dtn = dt / ntm;
+            dtm = dt - dtn * ntm;
+            off = dma_offsets<RT>(dtm * BM, dtn * BN, M, N, K, w, lane);
             bA = reinterpret_cast<const char*>(A);
             bW = reinterpret_cast<const char*>(W);
             bS = reinterpret_cast<const char*>(sbase);
@@ -410,14 +382,14 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
 
     // ---- compute side: the tile of the current segment of units
     TileRef cur;
-    {
-        const int t0 = (int)(u0 / NG);
-        cur.t = t0;
-        cur.g = (int)(u0 - (long long)t0 * NG);
-        const int tn = t0 / ntm;
-        cur.bm = (t0 - tn * ntm) * BM;
+    auto set_tile = [&](int t) __attribute__((always_inline)) {
+        const int tn = t / ntm;
+        cur.t = t;
+        cur.bm = (t - tn * ntm) * BM;
         cur.bn = tn * BN;
-    }
+    };
+    set_tile(t_first);
+    cur.g = g_first;
 
     // prologue: DMA of units 0..3, then the fragments of unit 0
     issue(0);
@@ -492,36 +464,22 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // One unit (one group of the current tile) from stage st; `first`: no earlier
-    // unit of this segment, so there is no row tile 3 awaiting its fold.
-    int i = 0;
-    auto unit = [&](bool first) __attribute__((always_inline)) {
-        const int st = i & (NS - 1);
-        TileRef x = cur;
-        TileRef xprev = cur;
-        if (GSUM) xprev.g = first ? -1 : cur.g - 1;   // -1: nothing to store
-        // row tile 0, with the unpack of this unit's weights and the fold of the
-        // previous unit's last tile
-        read_a(a_nxt, 1);
-        // (for the first unit of a segment accB and S2 are zero: the fold adds exact zeros)
-        step(a_cur, accA, accB, facc[3], 3, xprev, true, shi(S2));
-        S2 = scales2(sa2[0], sbr);
-        // row tile 1, fold of tile 0
-        read_a(a_cur, 2);
-        step(a_nxt, accB, accA, facc[0], 0, x, false, slo(S2));
-        // row tile 2, fold of tile 1
-        read_a(a_nxt, 3);
-        step(a_cur, accA, accB, facc[1], 1, x, false, shi(S2));
-        S2 = scales2(sa2[1], sbr);   // before the barrier: sa2, sbr are refilled with the next unit's after it
-        // row tile 3.  The DMA of unit i+1 has landed once at most the two younger
-        // units' loads are pending (three units in flight), and every wave has issued
-        // its last read of this stage (the barrier waits for LDS reads).  Near the
-        // end of the share fewer units are in flight; the first unit of a segment
-        // follows a flush, whose C stores are younger than that DMA and whose number
-        // depends on how many rows and columns of the tile exist; the group-sum
-        // variant stores as it goes.  In those cases no count bound is safe: drain.
-        if (GSUM || first || i + 3 >= n) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    int i = 0;   // the unit being computed
+    // Wait for the DMA of unit i + 1: at most the two younger units' loads may be
+    // pending (three units in flight).  Right after a flush its stores, at least 4 RT
+    // per wave, are younger still and need not be waited for.  Near the end of the share
+    // fewer units are in flight, and the group-sum variant stores as it goes: drain.
+    auto wait_next = [&](bool flushed) __attribute__((always_inline)) {
+        if (GSUM || i + 3 >= n) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else if (flushed) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DMA_PER_UNIT + 4 * RT) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * DMA_PER_UNIT) : "memory");
+    };
+    // The end of a unit's reads: the next unit's data has landed and every wave has
+    // issued its last read of this stage (the barrier waits for LDS reads); the stage is
+    // refilled and the next unit's operands are read.
+    auto turn = [&](v4i (&a_next)[4], bool flushed) __attribute__((always_inline)) {
+        const int st = i & (NS - 1);
+        wait_next(flushed);
         __syncthreads();
         if (i + 4 < n) {
             advance_dma();
@@ -529,70 +487,208 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
         }
         next_stage((st + 1) & (NS - 1));
         read_b();
-        read_a(a_cur, 0);
+        read_a(a_next, 0);
         read_s();
-        step(a_nxt, accB, accA, facc[2], 2, x, false, slo(S2));
+    };
+    // One unit (one group of the current tile) from stage i % NS; `first`: no earlier
+    // unit of this segment, so there is no last row tile awaiting its fold (accB and S2
+    // are zero and the fold adds exact zeros).
+    auto unit = [&](bool first) __attribute__((always_inline)) {
+        const bool flushed = first && i > 0;
+        TileRef x = cur;
+        TileRef xprev = cur;
+        if (GSUM) xprev.g = first ? -1 : cur.g - 1;   // -1: nothing to store
+        // row tile 0, with the unpack of this unit's weights and the fold of the
+        // previous unit's last tile
+        read_a(a_nxt, 1);
+        step(a_cur, accA, accB, facc[RT - 1], RT - 1, xprev, true, shi(S2));
+        S2 = scales2(sa2[0], sbr);
+        if constexpr (RT == 4) {
+            // row tile 1, fold of tile 0
+            read_a(a_cur, 2);
+            step(a_nxt, accB, accA, facc[0], 0, x, false, slo(S2));
+            // row tile 2, fold of tile 1
+            read_a(a_nxt, 3);
+            step(a_cur, accA, accB, facc[1], 1, x, false, shi(S2));
+            S2 = scales2(sa2[1], sbr);   // before the barrier: sa2, sbr are refilled with the next unit's after it
+        }
+        turn(a_cur, flushed);
+        // the last row tile, fold of the one before
+        constexpr int F = RT >= 2 ? RT - 2 : 0;
+        step(a_nxt, accB, accA, facc[F], F, x, false, slo(S2));
+        ++i;
+        if (GSUM) ++cur.g;
+    };
+    // RT = 1: one row tile per unit, the accumulators (and the scale products) taking
+    // turns from unit to unit.
+    auto unit1 = [&](v16i& acc, const v16i& prev, v32f& S, const v32f& Sprev, v4i (&a)[4], v4i (&a_next)[4],
+                     bool first) __attribute__((always_inline)) {
+        const bool flushed = first && i > 0;
+        TileRef xprev = cur;
+        if (GSUM) xprev.g = first ? -1 : cur.g - 1;
+        S = scales2(sa2[0], sbr);
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) unpack_ks(bu, bp, ks);
+        turn(a_next, flushed);
+        step(a, acc, prev, facc[0], 0, xprev, false, slo(Sprev));
         ++i;
         if (GSUM) ++cur.g;
     };
     // segments: the units of one tile within this workgroup's share
     while (i < n) {
-        const int g0 = (int)((u0 + i) % NG);
-        const int len = min(NG - g0, n - i);
-        if (GSUM) cur.g = g0;
+        const int len = seg_end(cur.t) - (i == 0 ? g_first : 0);
+        if (GSUM) cur.g = i == 0 ? g_first : 0;
         accB = zero16;
         S2 = zero32f;
-        for (int k = 0; k < len; k++) unit(k == 0);
-        // the segment's last row tile 3, then publish the segment
         TileRef xl = cur;
-        if (GSUM) xl.g = cur.g - 1;
+        if constexpr (RT == 1) {
+            v32f S1 = zero32f;
+            int k = 0;
+            for (; k + 1 < len; k += 2) {
+                unit1(accA, accB, S1, S2, a_cur, a_nxt, k == 0);
+                unit1(accB, accA, S2, S1, a_nxt, a_cur, false);
+            }
+            if (GSUM) xl.g = cur.g - 1;
+            if (k < len) {
+                unit1(accA, accB, S1, S2, a_cur, a_nxt, k == 0);
+                if (GSUM) xl.g = cur.g - 1;
 #pragma unroll
-        for (int q = 0; q < 4; q++) fold_q(facc[3], accB, shi(S2), 3, q, xl);
-        flush(cur);
+                for (int q = 0; q < 4; q++) fold_q(facc[0], accA, slo(S1), 0, q, xl);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; q++) fold_q(facc[0], accB, slo(S2), 0, q, xl);
+            }
+        } else {
+            for (int k = 0; k < len; k++) unit(k == 0);
+            if (GSUM) xl.g = cur.g - 1;
+            // the segment's last row tile, then publish the segment
+#pragma unroll
+            for (int q = 0; q < 4; q++) fold_q(facc[RT - 1], accB, shi(S2), RT - 1, q, xl);
+        }
+        flush(cur, len == NG);
         // the next unit's fragments, read again from its stage (still intact): the
         // copies read during the last unit are then dead across the flush, which
         // leaves the flush the registers it needs
         read_b();
         read_a(a_cur, 0);
         read_s();
-        // next tile
-        ++cur.t;
-        cur.bm += BM;
-        if (cur.bm >= ntm * BM) {
-            cur.bm = 0;
-            cur.bn += BN;
-        }
+        set_tile(next_tile(cur.t));
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// The split tiles: C = 1/16 of the sum of a tile's partials in workgroup order.  Block
+// (t, y) takes the 64 16-byte pieces 64 y.. of remainder tile t, one per thread: register
+// quad y / 8 of the GEMM's wave y % 8, i.e. 8 rows x 32 columns.  Up to four
+// contributors' loads are in flight per thread.
+// Its own launch, and not the last contributor of each tile within the GEMM: that
+// workgroup read up to 13 partials one round trip after another (8.9-19 us at the end of
+// a 20-34 us launch for 16-64 rows, 15.8 us at M=384 K=17408) while the others were done.
+template <int RT>
+__global__ __launch_bounds__(64) void gemm_combine_k(const float* __restrict__ part, float* __restrict__ C, int M,
+                                                      int N, int NG, GemmSched sch) {
+    constexpr int PB = 4;
+    const int t = blockIdx.x, tb = t * NG;
+    const int wf = owner_of(sch, tb), wl = owner_of(sch, tb + NG - 1);
+    if (wf == wl) return;                         // one workgroup's: already written
+    const int slot_f = 2 * wf + (range_start(sch, wf) == tb ? 0 : 1);
+    const int e = blockIdx.y * 64 + threadIdx.x;
+    const float4* src = reinterpret_cast<const float4*>(part) + e;
+    float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int v0 = wf; v0 <= wl; v0 += PB) {
+        float4 p[PB];
+#pragma unroll
+        for (int j = 0; j < PB; j++) {
+            const int v = min(v0 + j, wl);
+            p[j] = src[(size_t)(v == wf ? slot_f : 2 * v) * (Tile<RT>::PART_FLOATS / 4)];
+        }
+#pragma unroll
+        for (int j = 0; j < PB; j++)
+            if (v0 + j <= wl) {
+                f.x += p[j].x;
+                f.y += p[j].y;
+                f.z += p[j].z;
+                f.w += p[j].w;
+            }
+    }
+    // piece e: register quad k of thread e % NT of the GEMM's workgroup
+    const int k = e / NT, w = (e % NT) >> 6, lr = e & 31, lh = (e >> 5) & 1;
+    const int tn = t / sch.ntm, nn = tn * BN + 32 * w + lr;
+    const int m = (t - tn * sch.ntm) * Tile<RT>::BM + 32 * (k >> 2) + 8 * (k & 3) + 4 * lh;
+    if (nn >= N) return;
+    float* c = C + (size_t)m * N + nn;
+    if (m < M) c[0] = f.x * 0.0625f;
+    if (m + 1 < M) c[(size_t)N] = f.y * 0.0625f;
+    if (m + 2 < M) c[(size_t)N * 2] = f.z * 0.0625f;
+    if (m + 3 < M) c[(size_t)N * 3] = f.w * 0.0625f;
 }
 }  // namespace
 
 GemmPlan gemm_plan(int M, int N, int K, int cus) {
     GemmPlan p;
-    p.ntm = (M + BM - 1) / BM;
-    p.ntn = (N + BN - 1) / BN;
-    p.ntiles = p.ntm * p.ntn;
-    p.T = (long long)p.ntiles * (K / kGroup);
-    p.P = cus > 0 ? cus : 256;
-    if (p.T < p.P) p.P = (int)p.T;
-    p.part_bytes = (size_t)p.P * 2 * PART_FLOATS * sizeof(float);
-    p.cnt_bytes = (size_t)p.ntiles * sizeof(int);
+    const int NG = K / kGroup, ntn = (N + BN - 1) / BN, ncu = cus > 0 ? cus : 256;
+    p.rt = M <= 32 ? 1 : M <= 64 ? 2 : 4;
+    p.s.ntm = (M + 32 * p.rt - 1) / (32 * p.rt);
+    const int ntiles = p.s.ntm * ntn;
+    const long long T = (long long)ntiles * NG;
+    p.P = T < ncu ? (int)T : ncu;
+    p.s.full = ntiles / p.P;
+    p.s.rem = ntiles - p.s.full * p.P;
+    const int R = p.s.rem * NG;      // their units (rem < P; K = 128 NG < 2^31, so this fits)
+    // How many workgroups share the remainder tiles.  Every tile in S pieces on rem * S
+    // workgroups (S = 1: whole tiles, nothing to combine), or equal ranges on all of them
+    // (better balanced, but most workgroups then touch two tiles and leave two partials).
+    // Cost in us: the longest share, at the time a unit takes, and for a split the
+    // combining launch with its partials written and read.  Measured at M=1792 N=17408
+    // K=1152 (952 tiles of 9 groups, 184 left over): equal ranges 83.3 us a call, whole
+    // tiles 70.8.
+    const double unit_us = p.rt == 1 ? 0.6 : p.rt == 2 ? 0.87 : 1.36;
+    const double part_us = p.rt * (NT * 16 * sizeof(float)) / 4.5e6;
+    p.s.Pr = p.s.rem;
+    p.split = false;
+    double best = NG * unit_us;
+    const int smax = p.s.rem > 0 ? (p.P / p.s.rem < NG ? p.P / p.s.rem : NG) : 0;
+    for (int S = 2; S <= smax; S++) {
+        const double c = (NG + S - 1) / S * unit_us + 4.0 + (double)p.s.rem * S * part_us;
+        if (c < best) {
+            best = c;
+            p.s.Pr = p.s.rem * S;
+            p.split = true;
+        }
+    }
+    if (R >= p.P && p.s.rem > 0 &&
+        (double)((R + p.P - 1) / p.P) * unit_us + 4.0 + (double)(p.P + p.s.rem) * part_us < best) {
+        p.s.Pr = p.P;
+        p.split = true;
+    }
+    p.s.q = p.s.Pr > 0 ? R / p.s.Pr : 0;
+    p.s.r = p.s.Pr > 0 ? R % p.s.Pr : 0;
+    // two partials of a 128-row tile per workgroup, whatever the tile: one size serves
+    // every shape, so a call at a small shape leaves nothing to grow for a larger one
+    p.part_bytes = (size_t)p.P * 2 * Tile<4>::PART_FLOATS * sizeof(float);
     return p;
 }
 
 hipError_t launch_gemm_w4a8(float* C, int32_t* gsum, const int8_t* A, const uint32_t* W,
                             const float* sa, const float* sb, int M, int N, int K, const GemmPlan& p,
-                            float* part, int* cnt, hipStream_t st) {
-    if (gsum)
-        hipLaunchKernelGGL(gemm_w4a8_k<true>, dim3(p.P), dim3(NT), 0, st, A, W, sa, sb, C, gsum, part, cnt, M, N,
-                           K, p.ntm, p.T);
-    else
-        hipLaunchKernelGGL(gemm_w4a8_k<false>, dim3(p.P), dim3(NT), 0, st, A, W, sa, sb, C, gsum, part, cnt, M,
-                           N, K, p.ntm, p.T);
+                            float* part, hipStream_t st) {
+#define RT4_GEMM(R)                                                                                            \
+    if (gsum)                                                                                                  \
+        hipLaunchKernelGGL((gemm_w4a8_k<R, true>), dim3(p.P), dim3(NT), 0, st, A, W, sa, sb, C, gsum, part, M, N, K, p.s);  \
+    else                                                                                                       \
+        hipLaunchKernelGGL((gemm_w4a8_k<R, false>), dim3(p.P), dim3(NT), 0, st, A, W, sa, sb, C, gsum, part, M, N, K, p.s); \
+    if (p.split) hipLaunchKernelGGL(gemm_combine_k<R>, dim3(p.s.rem, 32 * R), dim3(64), 0, st, part, C, M, N, K / kGroup, p.s);
+    if (p.rt == 1) {
+        RT4_GEMM(1)
+    } else if (p.rt == 2) {
+        RT4_GEMM(2)
+    } else {
+        RT4_GEMM(4)
+    }
+#undef RT4_GEMM
     return hipGetLastError();
 }
 
-// Zero the split-tile counters once, when their workspace is (re)allocated.
+// Zero the split counters of a workspace once, when it is (re)allocated.
 __global__ void zero_i32_k(int* p, size_t n) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) p[i] = 0;

@@ -75,19 +75,26 @@ hipError_t launch_gemv_w4a4(float* y, const uint32_t* wq, const uint16_t* ws, co
 // C f32 [M][N] from int8 codes A [M][K] (interleaved), RT4 weights W [N][K/8],
 // group-major scales sa [K/128][M] and sb [K/128][N]; gsum (optional, tests)
 // receives the exact per-group int32 dot products [M][N][K/128].  The launch is
-// persistent (one workgroup per CU, equal shares of the (tile, group) units);
-// `part` and `cnt` are its split-tile workspace: part_bytes of partial sums and
-// cnt_bytes of counters that must be zero before the first launch (every launch
-// leaves them zero again).
+// persistent (one workgroup per CU).  `part` (part_bytes) is the workspace of the
+// partial sums of tiles that several workgroups share.
+struct GemmSched {
+    int ntm;       // row tiles
+    int full;      // whole tiles per workgroup; they follow the first rem tiles
+    int rem;       // tiles whose K groups are shared out evenly
+    int Pr;        // workgroups that share them
+    int q, r;      // their (tile, group) units, rem * K/128, over Pr: quotient and remainder
+};
 struct GemmPlan {
-    int ntm, ntn, ntiles, P;
-    long long T;
-    size_t part_bytes, cnt_bytes;
+    int rt;        // 32-row tiles per workgroup tile: 1, 2 or 4
+    int P;         // workgroups
+    GemmSched s;
+    bool split;    // some tile has several contributors: a combining launch follows
+    size_t part_bytes;
 };
 GemmPlan gemm_plan(int M, int N, int K, int cus);
 hipError_t launch_gemm_w4a8(float* C, int32_t* gsum, const int8_t* A, const uint32_t* W,
                             const float* sa, const float* sb, int M, int N, int K, const GemmPlan& plan,
-                            float* part, int* cnt, hipStream_t st);
+                            float* part, hipStream_t st);
 hipError_t launch_zero_i32(int* p, size_t n, hipStream_t st);
 
 // ---- int4-KV attention (attn.hip); head dim 256, Q/K groups of 128, V tiles of 64 keys

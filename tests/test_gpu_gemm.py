@@ -119,6 +119,33 @@ def test_gemm_reference_benchmark_shape(rt4, orc, torch_gpu):
     assert err < TIGHT and worst < 1e-5
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (2, 300, 640), (31, 256, 512), (32, 520, 1024), (33, 300, 1024), (63, 257, 384), (64, 512, 640), (65, 300, 512),
+    (16, 256, 17408),     # 136 workgroups share one tile, one group each
+    (1280, 8192, 256),    # 320 tiles on 256 CUs: one whole tile each after a shared remainder of 64
+    (128, 65536, 128),    # as many tiles as CUs: no remainder
+])
+def test_gemm_row_tiles_and_schedules(rt4, orc, torch_gpu, M, N, K):
+    """Row tiles of 32, 64 and 128 rows at their edges, and the shares of a tile count below, at and above the CU
+    count.  fp32 sums of K/128 terms in some order: rel L2 <= sqrt(K/128) * 2^-24 * 4 < 1e-6 for K <= 17408."""
+    print(f"case gemm row tiles M={M} N={N} K={K}", flush=True)
+    c, wq, ws, x = _case(torch_gpu, 41, M, N, K)
+    sb = rt4.make_group_major(ws, K)
+    xq, sc = rt4.quant_rows_i8(x)
+    out = torch_gpu.full((M, N), float("nan"), device="cuda")
+    y = host(rt4.gemm_w4a8_i8(wq, sb, xq, sc, out=out))
+    y2 = host(rt4.gemm_w4a8_i8(wq, sb, xq, sc))
+    assert np.array_equal(y.view(np.uint32), y2.view(np.uint32)), "repeated call differs"
+    assert not np.isnan(y).any()
+    rng = np.random.default_rng(M + N)
+    P = min(M * N, 8192)
+    pts = rng.choice(M * N, P, replace=False) if M * N < 1 << 20 else rng.integers(0, M * N, P)
+    mi, ni = (pts // N).astype(np.int32), (pts % N).astype(np.int32)
+    mi[:4], ni[:4] = [0, M - 1, 0, M - 1], [0, 0, N - 1, N - 1]
+    ref, _ = _oracle_points(orc, c, M, N, K, mi, ni)
+    assert rel_l2(y[mi, ni], ref) < TIGHT
+
+
 def test_gemm_dropin_small_c2_uses_library_scratch(rt4, orc, torch_gpu):
     """4*N < K: the recombined codes do not fit in c2, library scratch is used."""
     M, N, K = 128, 64, 1024
