@@ -20,9 +20,10 @@
  * memory; growth is by half at least.
  * Nothing is allocated while `stream` is being captured: a call that would
  * have to grow a scratch buffer then fails with RT4_E_CAPTURE, except that the
- * split GEMV and the attention prefill (automatic split count) fall back to
- * their unsplit forms, which need no workspace, and the prefill without room for
- * its staged K/V copy stages the tiles in every workgroup (same results).
+ * split GEMV falls back to its unsplit form, which needs no workspace, the attention
+ * prefill (automatic split count) to the largest split count whose workspace is there,
+ * down to one, and the prefill without room for its staged K/V copy stages the tiles in
+ * every workgroup (same results).
  *
  * Formats (docs/FORMAT.md:61-73 of the reference, unchanged here):
  *   wq   uint32 [N][K/8]   RT4 int4 weights: dword d holds k = 8d..8d+7, nibble e
@@ -256,10 +257,10 @@ int rt4_kv_append_v(uint32_t* vc, float* vsc, float* stage, const float* vf, int
  * algorithm: per 64-key tile P = clamp(int(7 exp(s - m_tile) + 0.5), 0, 7) and
  * online rescaling (the running reference moves only when a tile's max exceeds
  * it by more than a factor 2^8: the same O and L, rounded differently).  Query
- * row i has position off + i.  K/V are staged once per call (codes unpacked into
- * the MFMA operand bytes, 32 KB per key tile and KV head of library scratch; at
- * most 4 GiB, beyond which each workgroup stages its own tiles), then DMA'd into
- * LDS by the workgroups.  Replaces the prefill
+ * row i has position off + i.  Where each workgroup has many tiles, K/V are staged
+ * once per call (codes unpacked into the MFMA operand bytes, 32 KB per key tile and
+ * KV head of library scratch; at most 4 GiB), then DMA'd into LDS by the workgroups;
+ * otherwise each workgroup stages its own tiles (same results).  Replaces the prefill
  * branch of k_attention (src/kernels.h:81, src/k_fa.hip:282-300; kernel fa_int4,
  * kernels/flash_attn_core.h:74-435).  n_q % 64 == 0, kv_cap % 64 == 0,
  * n_tile * 64 <= kv_cap, kv_cap <= 16777152 (2^24 - 64: one KV head's cache is
@@ -270,11 +271,12 @@ int rt4_attention_prefill(float* out, const uint32_t* qq, const float* qsc, cons
 
 /* Same, with an explicit number of KV splits per (64-row query block, head)
  * (tuning and tests; 0 selects the default that balances the grid over the
- * device's CUs).  With more than one split each split writes its partial state
- * (unnormalised output, running max, denominator) to library scratch (grown
- * with hipMalloc, with one counter per (query block, head)), and the split that
- * finishes last for a (query block, head) combines them in split order within
- * the same launch. */
+ * device's CUs; at most 64).  With more than one split each split writes its
+ * partial state (unnormalised output, running max, denominator) to library scratch
+ * (grown with hipMalloc), and the partial states are combined in split order: by the
+ * split that finishes last for a (query block, head) within the same launch (up to 4
+ * splits of a large grid; one counter per (query block, head)), else by a launch of
+ * their own. */
 int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, const uint32_t* kc,
                               const float* ksc, const uint32_t* vc, const float* vsc, int n_q, int n_kv,
                               int off, int n_tile, int n_heads, int ratio, int kv_cap, int kv_splits,

@@ -52,13 +52,18 @@
 // Row max over a query's 64 keys is 15 in-lane ops plus two cross-lane steps
 // (xor 16, xor 32).  The K/V tiles reach LDS in MFMA operand order (16 bytes per
 // (subtile, group, half, lane)), so the waves only issue ds_read_b128 of ready
-// operands.  A pre-pass (fa_expand_kv_k) unpacks every tile once per call into a
-// copy in memory with exactly that layout, and the workgroups move each tile into
-// LDS with global_load_lds_dwordx4 (no registers, no unpacking, no LDS stores):
-// unpacking in every workgroup repeated it once per query block and split, about a
-// tenth of the kernel at C4.  Without room for the copy (graph capture before the
-// first eager call, or a copy beyond 4 GiB) each workgroup stages its tiles itself
-// from the packed cache, with the same bytes.  Tiles past the workgroup's last query
+// operands.  Where workgroups have many tiles (fa_plan), a pre-pass (fa_expand_kv_k)
+// unpacks every tile once per call into a copy in memory with exactly that layout, and
+// the workgroups move each tile into LDS with global_load_lds_dwordx4 (no registers, no
+// unpacking, no LDS stores): unpacking in every workgroup repeated it once per query
+// block and split, about a tenth of the kernel at C4.  With few tiles a workgroup, or
+// without room for the copy (graph capture before the first eager call, or a copy beyond
+// 4 GiB), each workgroup stages its tiles itself from the packed cache, with the same
+// bytes.  The KV range is split over workgroups until the grid fills the CUs (fa_plan),
+// down to three tiles a workgroup; a workgroup starts with one memory round trip (Q and
+// the first tiles' loads together) and converts Q by table look-up (v_perm_b32) while
+// the tiles arrive (both: C4 645 -> 639 us, 43 rows over 4096 keys 26.2 -> 25.2).
+// Tiles past the workgroup's last query
 // position are skipped: the reference processes them but every entry is masked,
 // which leaves its state bit-for-bit unchanged.  The tile loop is a two-tile
 // pipeline (S and P of the next tile beside the PV product of the current one;
@@ -105,12 +110,15 @@ __device__ __forceinline__ v8i cat8(v4i lo, v4i hi) {
 // nibbles 0, 2, 4, 6 (even) or 1, 3, 5, 7 (odd) as the bytes c + 8 = E4M3 of (c + 8)·2^-9.
 __device__ __forceinline__ uint32_t even_e4m3(uint32_t w8) { return w8 & 0x0F0F0F0Fu; }
 __device__ __forceinline__ uint32_t odd_e4m3(uint32_t w8) { return (w8 >> 4) & 0x0F0F0F0Fu; }
-// E4M3 encoding of an integer -8..8: magnitudes 0..7 are the bytes 00 38 40 44 48
-// 4A 4C 4E (exponent bias 7, 3 mantissa bits), 8 is 0x50; sign in bit 7.
-__device__ __forceinline__ uint32_t e4m3_of_int(int c) {
-    const uint32_t m = (uint32_t)(c < 0 ? -c : c);
-    const uint32_t b = m < 8 ? (uint32_t)(0x4E4C4A4844403800ull >> (8 * m)) & 0xFFu : 0x50u;
-    return b | (c < 0 ? 0x80u : 0u);
+// Exact E4M3 bytes of four signed codes held in the low nibbles of x's bytes (the high
+// nibbles are ignored): v_perm_b32 looks the codes 0..7 and -8..-1 up in two 8-byte
+// tables (exponent bias 7, 3 mantissa bits: 1 = 38, 2 = 40, 3 = 44, ..., 8 = 50), and bit
+// 3 of each nibble chooses.
+__device__ __forceinline__ uint32_t e4m3_of_codes(uint32_t x) {
+    const uint32_t sel = x & 0x07070707u, neg = (x >> 3) & 0x01010101u, m = (neg << 8) - neg;
+    const uint32_t pos = __builtin_amdgcn_perm(0x4E4C4A48u, 0x44403800u, sel);   // codes 4..7, 0..3
+    const uint32_t ngt = __builtin_amdgcn_perm(0xB8C0C4C8u, 0xCACCCED0u, sel);   // codes -4..-1, -8..-5
+    return (pos & ~m) | (ngt & m);
 }
 
 // Key order within a 16-key subtile: output register r of lane group G holds key
@@ -202,8 +210,11 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
     // lane l, register 4kt + r, the operand of lane 16kt + 4(l >> 4) + r, so lane j
     // supplies the key of register j & 3 of lane group (j >> 2) & 3 in subtile j >> 4
     const int kslot = 16 * G + key_of_slot((lane >> 2) & 3, lane & 3);
-    const int head = blockIdx.y, vh = head / ratio;
-    const int q0 = blockIdx.x * QROWS;
+    // heads fastest, then the query blocks from the last (most tiles) to the first: with
+    // fewer workgroups than slots the long ones get a CU each and the short ones join them
+    const int head = blockIdx.x, vh = head / ratio;
+    const int qb = gridDim.y - 1 - blockIdx.y;
+    const int q0 = qb * QROWS;
     const int qrow = q0 + 16 * w + qi;
     qq += (size_t)head * n_q * KDW;
     qsc += (size_t)head * 2 * n_q;
@@ -222,34 +233,33 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
 
     // Resident Q operand of group g: dims 128g + 32G .. +31, the 4 code dwords w_m
     // (dims 8m..8m+7 of that range) as E4M3 bytes in the order even(w0) odd(w0)
-    // even(w1) ... odd(w3), the order the K operand bytes are staged in.  cS[g] =
+    // even(w1) ... odd(w3), the order the K operand bytes are staged in.  cS0, cS1 =
     // -8·Σq·2^-9 over the group's 128 dims takes the K offset back off.
     v8i qop[2];
-    float cS[2];
+    v4f cS0, cS1;
+    uint4 qraw[2];
 #pragma unroll
-    for (int g = 0; g < 2; g++) {
-        const uint4 wd = *reinterpret_cast<const uint4*>(qq + (size_t)qrow * KDW + 16 * g + 4 * G);
-        const uint32_t w[4] = {wd.x, wd.y, wd.z, wd.w};
-        int qs = 0;
+    for (int g = 0; g < 2; g++) qraw[g] = *reinterpret_cast<const uint4*>(qq + (size_t)qrow * KDW + 16 * g + 4 * G);
+    auto make_q = [&]() __attribute__((always_inline)) {
+        int qs[2] = {0, 0};
 #pragma unroll
-        for (int m = 0; m < 4; m++) {
-            uint32_t ev = 0, od = 0;
+        for (int g = 0; g < 2; g++) {
+            const uint32_t w[4] = {qraw[g].x, qraw[g].y, qraw[g].z, qraw[g].w};
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int ce = sext4(w[m], 2 * j), co = sext4(w[m], 2 * j + 1);
-                qs += ce + co;
-                ev |= e4m3_of_int(ce) << (8 * j);
-                od |= e4m3_of_int(co) << (8 * j);
+            for (int m = 0; m < 4; m++) {
+                qs[g] = __builtin_amdgcn_sdot8((int)w[m], 0x11111111, qs[g], false);
+                qop[g][2 * m] = (int)e4m3_of_codes(w[m]);
+                qop[g][2 * m + 1] = (int)e4m3_of_codes(w[m] >> 4);
             }
-            qop[g][2 * m] = (int)ev;
-            qop[g][2 * m + 1] = (int)od;
+            qs[g] += __shfl_xor(qs[g], 16);
+            qs[g] += __shfl_xor(qs[g], 32);
         }
-        qs += __shfl_xor(qs, 16);
-        qs += __shfl_xor(qs, 32);
-        cS[g] = (float)(-8 * qs) * (1.f / 512.f);
-    }
-    // S in log2 units: fold log2(e) and the 2^9 of the offset K operand into the Q scales
-    const float A0 = qsc[qrow] * (L2E * 512.f), A1 = qsc[n_q + qrow] * (L2E * 512.f);
+        const float c0 = (float)(-8 * qs[0]) * (1.f / 512.f), c1 = (float)(-8 * qs[1]) * (1.f / 512.f);
+        cS0 = v4f{c0, c0, c0, c0};
+        cS1 = v4f{c1, c1, c1, c1};
+    };
+    // S in log2 units: log2(e) and the 2^9 of the offset K operand go into the Q scales
+    float A0 = qsc[qrow], A1 = qsc[n_q + qrow];
 
     float O[16][4];
 #pragma unroll
@@ -354,7 +364,6 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
         dma16<3072>(lane * 16 + (4 * w + 3) * 1024, src, dst);
     };
 
-    const v4f cS0 = {cS[0], cS[0], cS[0], cS[0]}, cS1 = {cS[1], cS[1], cS[1], cS[1]};
     // front of tile t (K in buffer b): S^T = K Q^T for the 4 subtiles of 16 keys,
     // the causal mask (MASK: the tile may reach past a row of this workgroup), the
     // tile max m of each row, the P codes as the PV operand and -8·ΣP·2^-18.
@@ -526,7 +535,9 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
         // tiles from t_mask on may reach past the position of some row of this
         // workgroup (row q0 of wave 0 is the first): their front takes the masked form
         const int t_mask = (off + q0 + 1) / BNK;
-        StageK sk;
+        // The first tiles' loads are issued together with Q's (above) and its conversion
+        // done while they arrive: one memory round trip at the start.
+        StageK sk, sk1;
         StageV sv;
         if constexpr (DMA) {
             dma_k(t0, t0 & 1);
@@ -535,10 +546,14 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
         }
         load_k(sk, t0);
         load_v(sv, t0);
+        load_k(sk1, t0 + 1);
+        asm volatile("" ::: "memory");
+        make_q();
+        A0 *= L2E * 512.f;
+        A1 *= L2E * 512.f;
         store_k(sk, t0 & 1, t0);
         store_v(sv, t0 & 1, t0);
-        load_k(sk, t0 + 1);
-        store_k(sk, (t0 + 1) & 1, t0 + 1);
+        store_k(sk1, (t0 + 1) & 1, t0 + 1);
         load_k(sk, t0 + 2);
         load_v(sv, t0 + 1);
         if constexpr (DMA) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -600,15 +615,14 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
         // -- and re-arms the counter for the next call.  No workgroup waits for
         // another.
         constexpr int kSc1 = 16;    // cache policy: sc1
-        constexpr int kFastSplits = 4;   // split counts combined with loads issued in bulk
-        const int item = head * gridDim.x + blockIdx.x;
+        const int item = head * gridDim.y + qb;
         // this query block's 64 rows of split s: O [64][HD] and (m, L) [64]
         auto o_rsrc = [&](int s) {
-            return __builtin_amdgcn_make_buffer_rsrc(opart + (((size_t)s * gridDim.y + head) * n_q + q0) * HD, 0,
+            return __builtin_amdgcn_make_buffer_rsrc(opart + (((size_t)s * gridDim.x + head) * n_q + q0) * HD, 0,
                                                      QROWS * HD * 4, kRsrcW3);
         };
         auto ml_rsrc = [&](int s) {
-            return __builtin_amdgcn_make_buffer_rsrc(mlpart + ((size_t)s * gridDim.y + head) * n_q + q0, 0,
+            return __builtin_amdgcn_make_buffer_rsrc(mlpart + ((size_t)s * gridDim.x + head) * n_q + q0, 0,
                                                      QROWS * 8, kRsrcW3);
         };
         const int ooff = ((16 * w + qi) * HD + 4 * G) * 4;   // this lane's first 16 bytes in a block
@@ -625,6 +639,7 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
                 __builtin_amdgcn_raw_buffer_store_b64(v2u{__float_as_uint(rref), __float_as_uint(L)}, ml_rsrc(split),
                                                       moff, 0, kSc1);
         }
+        if (!cnt) return;                        // fa_combine_k sums the splits
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (tid == 0)
@@ -641,69 +656,50 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
 #pragma unroll
                 for (int r = 0; r < 4; r++) o[dt][r] = 0.f;
             float l = 0.f;
-            if (nsplit <= kFastSplits) {
-                // All loads of a round are issued before any is used: every split's
-                // (m, L) in one round, then the partial O in four rounds of 64 dims,
-                // each holding that quarter of every split (5 memory round trips in
-                // place of 2·nsplit + 1 dependent ones).  This workgroup's own split
-                // is read back like the others (its stores completed at vmcnt(0)
-                // above).  The sums run in split order, as in the general path.
-                float2 ml[kFastSplits];
+            // All loads of a round are issued before any is used: every split's
+            // (m, L) in one round, then the partial O in four rounds of 64 dims,
+            // each holding that quarter of every split (5 memory round trips in
+            // place of 2·nsplit + 1 dependent ones).  This workgroup's own split
+            // is read back like the others (its stores completed at vmcnt(0)
+            // above).  The sums run in split order.
+            float2 ml[kFaInlineSplits];
 #pragma unroll
-                for (int s = 0; s < kFastSplits; s++)
-                    if (s < nsplit) ml[s] = ml_of(s);
-                float Mx = -__builtin_inff();
+            for (int s = 0; s < kFaInlineSplits; s++)
+                if (s < nsplit) ml[s] = ml_of(s);
+            float Mx = -__builtin_inff();
 #pragma unroll
-                for (int s = 0; s < kFastSplits; s++)
-                    if (s < nsplit) Mx = fmaxf(Mx, ml[s].x);
-                float a[kFastSplits];
+            for (int s = 0; s < kFaInlineSplits; s++)
+                if (s < nsplit) Mx = fmaxf(Mx, ml[s].x);
+            float a[kFaInlineSplits];
 #pragma unroll
-                for (int s = 0; s < kFastSplits; s++)
+            for (int s = 0; s < kFaInlineSplits; s++)
+                if (s < nsplit) {
+                    a[s] = exp2f(ml[s].x - Mx);
+                    l = fmaf(a[s], ml[s].y, l);
+                }
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                v4u b[kFaInlineSplits][4];
+#pragma unroll
+                for (int s = 0; s < kFaInlineSplits; s++)
                     if (s < nsplit) {
-                        a[s] = exp2f(ml[s].x - Mx);
-                        l = fmaf(a[s], ml[s].y, l);
+                        const __amdgpu_buffer_rsrc_t rs = o_rsrc(s);
+#pragma unroll
+                        for (int d = 0; d < 4; d++)
+                            b[s][d] = __builtin_amdgcn_raw_buffer_load_b128(rs, ooff + (4 * c + d) * 64, 0, kSc1);
                     }
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    v4u b[kFastSplits][4];
+                for (int s = 0; s < kFaInlineSplits; s++)
+                    if (s < nsplit) {
 #pragma unroll
-                    for (int s = 0; s < kFastSplits; s++)
-                        if (s < nsplit) {
-                            const __amdgpu_buffer_rsrc_t rs = o_rsrc(s);
-#pragma unroll
-                            for (int d = 0; d < 4; d++)
-                                b[s][d] = __builtin_amdgcn_raw_buffer_load_b128(rs, ooff + (4 * c + d) * 64, 0, kSc1);
+                        for (int d = 0; d < 4; d++) {
+                            const int dt = 4 * c + d;
+                            o[dt][0] = fmaf(a[s], __uint_as_float(b[s][d].x), o[dt][0]);
+                            o[dt][1] = fmaf(a[s], __uint_as_float(b[s][d].y), o[dt][1]);
+                            o[dt][2] = fmaf(a[s], __uint_as_float(b[s][d].z), o[dt][2]);
+                            o[dt][3] = fmaf(a[s], __uint_as_float(b[s][d].w), o[dt][3]);
                         }
-#pragma unroll
-                    for (int s = 0; s < kFastSplits; s++)
-                        if (s < nsplit) {
-#pragma unroll
-                            for (int d = 0; d < 4; d++) {
-                                const int dt = 4 * c + d;
-                                o[dt][0] = fmaf(a[s], __uint_as_float(b[s][d].x), o[dt][0]);
-                                o[dt][1] = fmaf(a[s], __uint_as_float(b[s][d].y), o[dt][1]);
-                                o[dt][2] = fmaf(a[s], __uint_as_float(b[s][d].z), o[dt][2]);
-                                o[dt][3] = fmaf(a[s], __uint_as_float(b[s][d].w), o[dt][3]);
-                            }
-                        }
-                }
-            } else {
-                float Mx = -__builtin_inff();
-                for (int s = 0; s < nsplit; s++) Mx = fmaxf(Mx, ml_of(s).x);
-                for (int s = 0; s < nsplit; s++) {
-                    const float2 ml = ml_of(s);
-                    const float a = exp2f(ml.x - Mx);
-                    const __amdgpu_buffer_rsrc_t rs = o_rsrc(s);
-#pragma unroll
-                    for (int dt = 0; dt < 16; dt++) {
-                        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rs, ooff + dt * 64, 0, kSc1);
-                        o[dt][0] = fmaf(a, __uint_as_float(v.x), o[dt][0]);
-                        o[dt][1] = fmaf(a, __uint_as_float(v.y), o[dt][1]);
-                        o[dt][2] = fmaf(a, __uint_as_float(v.z), o[dt][2]);
-                        o[dt][3] = fmaf(a, __uint_as_float(v.w), o[dt][3]);
                     }
-                    l = fmaf(a, ml.y, l);
-                }
             }
             float* orow = out + (size_t)qrow * HD + 4 * G;
 #pragma unroll
@@ -714,6 +710,41 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
             if (tid == 0) __hip_atomic_store(cnt + item, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+}
+
+// Sum of the KV splits' partial states (fa_plan says when: more than kFaInlineSplits of
+// them, or a grid of one round, where the last split would do it alone at the end, a
+// workgroup reading every partial of 64 rows: of a 44 us call at 64 rows, 24 heads and
+// 4096 keys in 8 splits that was ~13): one wave per half row, two dims a lane.  M = max_s m_s, a_s = 2^(m_s - M), out = Σ_s a_s O_s / Σ_s a_s L_s, the
+// sums in split order.  PB splits' loads are in flight at a time.
+template <int PB>
+__global__ __launch_bounds__(256) void fa_combine_k(const float* __restrict__ opart, const float2* __restrict__ mlpart,
+                                                    float* __restrict__ out, int rows, int nsplit) {
+    const int lane = threadIdx.x & 63, w = uniform(threadIdx.x >> 6);
+    const int row = blockIdx.x * 2 + (w >> 1), d = 128 * (w & 1) + 2 * lane;   // row over heads and queries
+    // lane s holds split s (at most 64)
+    const float2 ml = lane < nsplit ? mlpart[(size_t)lane * rows + row] : make_float2(-__builtin_inff(), 0.f);
+    const float M = run_max<64>(ml.x);
+    const float a = lane < nsplit ? exp2f(ml.x - M) : 0.f;
+    float l = a * ml.y;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+    const float2* src = reinterpret_cast<const float2*>(opart + (size_t)row * HD + d);
+    float2 acc = make_float2(0.f, 0.f);
+    for (int s0 = 0; s0 < nsplit; s0 += PB) {
+        float2 v[PB];
+#pragma unroll
+        for (int j = 0; j < PB; j++) v[j] = src[(size_t)min(s0 + j, nsplit - 1) * rows * (HD / 2)];
+#pragma unroll
+        for (int j = 0; j < PB; j++)
+            if (s0 + j < nsplit) {
+                const float as = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a), s0 + j));
+                acc.x = fmaf(as, v[j].x, acc.x);
+                acc.y = fmaf(as, v[j].y, acc.y);
+            }
+    }
+    *reinterpret_cast<float2*>(out + (size_t)row * HD + d) =
+        make_float2(l > 0.f ? acc.x / l : 0.f, l > 0.f ? acc.y / l : 0.f);
 }
 
 // Staged K/V blocks of every tile of every KV head, for the DMA path: the kernel's
@@ -749,22 +780,46 @@ __global__ __launch_bounds__(256) void fa_expand_kv_k(const uint32_t* __restrict
 
 // -------------------------------------------------------------- launchers --
 
-int fa_splits(int n_q, int n_heads, int n_tile, int cus) {
-    // workgroups resident per CU: LDS (double-buffered operands) allows two
-    const int slots = (cus > 0 ? cus : 256) * 2;
-    const int items = (n_q / QROWS) * n_heads;
-    int best = 1;
-    double best_eff = 0.0;
-    for (int s = 1; s <= 8; s++) {
-        if (s > 1 && n_tile / s < 8) break;          // keep at least 8 tiles per split
+FaPlan fa_plan(int n_q, int n_heads, int ratio, int off, int n_tile, int cus, int kv_splits) {
+    // The cheapest split count by a cost model (us) fitted to the sweep below: a tile takes
+    // 1.3 us in a workgroup that has its CU to itself and 1.6 where two share one (LDS
+    // allows two), in as many rounds as the grid needs; ~6 us to start and end; the
+    // combining launch 3.5 us and the partials (64 KB a workgroup, written and read) 0.025
+    // each, of which most hides when the last splits combine while others still run.
+    // Measured (one layer, 24 heads over 4 KV heads unless noted; us for the start's rule
+    // of at most 8 splits of at least 8 tiles, balancing rounds only -> this one): 43
+    // rows over 4096 keys 44 -> 25 (10 splits), 100 rows 49 -> 33, 64 rows over 1024 keys
+    // 28.5 -> 17 (6), 6 rows over 25088 keys with 6 heads over one KV head 92 -> 28 (42),
+    // 9 rows over 9472 with 8 over 8 60 -> 23 (32); C4 keeps its 4.
+    cus = cus > 0 ? cus : 256;
+    const int items = n_q / QROWS * n_heads, slots = 2 * cus;
+    const int last = (off + n_q - 1) / BNK + 1, nt = last < n_tile ? last : n_tile;   // tiles of the last block
+    FaPlan p{1, false, false};
+    double best = 0.0;
+    for (int s = 1; s <= kFaMaxSplits && s <= nt; s++) {
+        if (kv_splits > 0 && s != kv_splits && !(s == 1)) continue;
         const long long blocks = (long long)items * s;
-        const double eff = (double)blocks / ((double)slots * (double)((blocks + slots - 1) / slots));
-        if (eff > best_eff + 0.02) {
-            best_eff = eff;
-            best = s;
+        const double rounds = (double)((blocks + slots - 1) / slots);
+        const bool in = s > 1 && s <= kFaInlineSplits && blocks > slots;
+        double c = (double)((nt + s - 1) / s) * rounds * (blocks <= cus ? 1.3 : 1.6);
+        if (s > 1) c += 3.5 + (double)blocks * (in ? 0.006 : 0.025);
+        if (s == 1 || s == kv_splits || (kv_splits == 0 && c < best)) {
+            best = c;
+            p.nsplit = s;
+            p.inline_combine = in;
         }
     }
-    return best;
+    if (kv_splits > 0 && p.nsplit != kv_splits) {       // more splits than tiles: some are empty
+        p.nsplit = kv_splits;
+        p.inline_combine = kv_splits <= kFaInlineSplits && (long long)items * kv_splits > slots;
+    }
+    // Stage K/V once for all (a launch, ~4 us and 6.5 ns a tile and KV head), or in every
+    // workgroup, which costs it 0.2 us a tile (0.4 where two share a CU): 43 rows over 4096
+    // keys 29 us staged, 25 not; C4 639 staged, 758 not.
+    const long long blocks = (long long)items * p.nsplit;
+    const double visits = (double)((nt + p.nsplit - 1) / p.nsplit) * (double)((blocks + slots - 1) / slots);
+    p.staged = visits * (blocks <= cus ? 0.2 : 0.4) > 4.0 + 0.0065 * (double)n_tile * (n_heads / ratio);
+    return p;
 }
 
 size_t fa_part_bytes(int n_q, int n_heads, int nsplit) {
@@ -785,20 +840,28 @@ hipError_t launch_fa_int4(float* out, const uint32_t* qq, const float* qsc, cons
                           hipStream_t st) {
     float* opart = part;
     float2* mlpart = part ? reinterpret_cast<float2*>(part + (size_t)nsplit * n_heads * n_q * HD) : nullptr;
-    const dim3 grid(n_q / QROWS, n_heads, nsplit);
+    const dim3 grid(n_heads, n_q / QROWS, nsplit);
+    hipError_t e;
     if (!kvx) {
         hipLaunchKernelGGL(fa_int4_k<false>, grid, dim3(NTA), 0, st, qq, qsc, kc, ksc, vc, vsc, out, n_q, n_kv, off,
                            n_tile, ratio, kv_cap, nsplit, opart, mlpart, cnt, nullptr, nullptr);
-        return hipGetLastError();
+    } else {
+        const int kvh = n_heads / ratio;
+        unsigned char* kx = static_cast<unsigned char*>(kvx);
+        unsigned char* vx = kx + (size_t)kvh * n_tile * KU_BYTES;
+        hipLaunchKernelGGL(fa_expand_kv_k, dim3(n_tile, kvh, 2), dim3(256), 0, st, kc, vc, kx, vx, n_kv, n_tile, kv_cap);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        hipLaunchKernelGGL(fa_int4_k<true>, grid, dim3(NTA), 0, st, qq, qsc, kc, ksc, vc, vsc, out, n_q, n_kv, off,
+                           n_tile, ratio, kv_cap, nsplit, opart, mlpart, cnt, kx, vx);
     }
-    const int kvh = n_heads / ratio;
-    unsigned char* kx = static_cast<unsigned char*>(kvx);
-    unsigned char* vx = kx + (size_t)kvh * n_tile * KU_BYTES;
-    hipLaunchKernelGGL(fa_expand_kv_k, dim3(n_tile, kvh, 2), dim3(256), 0, st, kc, vc, kx, vx, n_kv, n_tile, kv_cap);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(fa_int4_k<true>, grid, dim3(NTA), 0, st, qq, qsc, kc, ksc, vc, vsc, out, n_q, n_kv, off,
-                       n_tile, ratio, kv_cap, nsplit, opart, mlpart, cnt, kx, vx);
+    if ((e = hipGetLastError()) != hipSuccess || nsplit == 1 || cnt) return e;
+#define RT4_FC(PB) \
+    hipLaunchKernelGGL(fa_combine_k<PB>, dim3(n_heads * n_q / 2), dim3(256), 0, st, opart, mlpart, out, n_heads * n_q, nsplit)
+    if (nsplit <= 2) RT4_FC(2);
+    else if (nsplit <= 4) RT4_FC(4);
+    else if (nsplit <= 8) RT4_FC(8);
+    else RT4_FC(16);
+#undef RT4_FC
     return hipGetLastError();
 }
 

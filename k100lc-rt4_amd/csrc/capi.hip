@@ -714,28 +714,35 @@ int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, 
     int cus = 0, rc = device_cus(&cus);
     if (rc) return rc;
     hipStream_t st = as_stream(stream);
-    int nsplit = kv_splits > 0 ? kv_splits : rt4::fa_splits(n_q, n_heads, n_tile, cus);
+    rt4::FaPlan plan = rt4::fa_plan(n_q, n_heads, ratio, off, n_tile, cus, kv_splits);
     // Under graph capture an automatic split count that would need a larger
-    // workspace falls back to one split (no workspace; same algorithm, the fp32
-    // sums of O and L in one order instead of a combine of partial ranges).
-    if (nsplit > 1 && kv_splits == 0 && capturing(st) &&
-        !(scratch_has(kSlotAttnPart, rt4::fa_part_bytes(n_q, n_heads, nsplit)) &&
-          scratch_has(kSlotAttnCnt, rt4::fa_cnt_bytes(n_q, n_heads, nsplit))))
-        nsplit = 1;
+    // workspace falls back to the largest count whose workspace is there, down to one
+    // split, which needs none (same algorithm, the fp32 sums of O and L in another order).
+    if (kv_splits == 0 && plan.nsplit > 1 && capturing(st)) {
+        auto fits = [&](const rt4::FaPlan& p) {
+            return scratch_has(kSlotAttnPart, rt4::fa_part_bytes(n_q, n_heads, p.nsplit)) &&
+                   (!p.inline_combine || scratch_has(kSlotAttnCnt, rt4::fa_cnt_bytes(n_q, n_heads, p.nsplit)));
+        };
+        while (plan.nsplit > 1 && !fits(plan))
+            plan = rt4::fa_plan(n_q, n_heads, ratio, off, n_tile, cus, plan.nsplit - 1);
+    }
     void *part = nullptr, *cnt = nullptr;
-    if (nsplit > 1 && ((rc = lib_scratch(kSlotAttnPart, rt4::fa_part_bytes(n_q, n_heads, nsplit), &part, st)) ||
-                       (rc = lib_scratch(kSlotAttnCnt, rt4::fa_cnt_bytes(n_q, n_heads, nsplit), &cnt, st, true))))
+    if (plan.nsplit > 1 &&
+        ((rc = lib_scratch(kSlotAttnPart, rt4::fa_part_bytes(n_q, n_heads, plan.nsplit), &part, st)) ||
+         (plan.inline_combine &&
+          (rc = lib_scratch(kSlotAttnCnt, rt4::fa_cnt_bytes(n_q, n_heads, plan.nsplit), &cnt, st, true)))))
         return rc;
     // The staged K/V copy for the DMA form (one staging pass per call instead of per
-    // workgroup), up to kMaxKvxBytes; beyond that, or under capture while the copy
-    // would have to grow, each workgroup stages its own tiles (same results).
+    // workgroup), where it pays and up to kMaxKvxBytes; beyond that, or under capture while
+    // the copy would have to grow, each workgroup stages its own tiles (same results).
     const size_t xb = rt4::fa_kvx_bytes(n_heads, ratio, n_tile);
     void* kvx = nullptr;
-    if (xb <= kMaxKvxBytes && !(capturing(st) && !scratch_has(kSlotAttnKV, xb)) &&
+    if (plan.staged && xb <= kMaxKvxBytes && !(capturing(st) && !scratch_has(kSlotAttnKV, xb)) &&
         (rc = lib_scratch(kSlotAttnKV, xb, &kvx, st)))
         return rc;
     return hip_status(rt4::launch_fa_int4(out, qq, qsc, kc, ksc, vc, vsc, n_q, n_kv, off, n_tile, n_heads, ratio,
-                                          kv_cap, nsplit, static_cast<float*>(part), static_cast<int*>(cnt), kvx, st),
+                                          kv_cap, plan.nsplit, static_cast<float*>(part), static_cast<int*>(cnt), kvx,
+                                          st),
                       "k_attention launch");
 }
 

@@ -104,16 +104,24 @@ hipError_t launch_kv_append_k(uint32_t* kc, float* ksc, const float* kf, int t0,
                               int kv_total, hipStream_t st);
 hipError_t launch_kv_append_v(uint32_t* vc, float* vsc, float* stage, const float* vf, int t0, int T, int H,
                               int D, int BG, int kv_total, hipStream_t st);
-// KV splits per (query block, head) that balance the grid over `cus` CUs, and
-// the workspace they need (0 for one split): partial states, and one counter per
-// (query block, head) that must be zero before the first launch (every launch
-// leaves them zero again).
-int fa_splits(int n_q, int n_heads, int n_tile, int cus);
+// How a prefill call runs: KV splits per (query block, head); whether the split that
+// finishes last combines them in the same launch (at most kFaInlineSplits) or a launch
+// of its own does; whether K/V are staged once for all workgroups.  kv_splits > 0 fixes
+// the count.  The workspace (0 for one split): partial states, and for the combine in
+// the same launch one counter per (query block, head) that must be zero before the first
+// launch (every launch leaves them zero again).
+constexpr int kFaMaxSplits = 64, kFaInlineSplits = 4;
+struct FaPlan {
+    int nsplit;
+    bool inline_combine, staged;
+};
+FaPlan fa_plan(int n_q, int n_heads, int ratio, int off, int n_tile, int cus, int kv_splits);
 size_t fa_part_bytes(int n_q, int n_heads, int nsplit);
 size_t fa_cnt_bytes(int n_q, int n_heads, int nsplit);
 // Bytes of the staged K/V copy the DMA form of the prefill reads (two 16 KB blocks
 // per tile and KV head).  launch_fa_int4 with kvx (that many bytes) fills it and runs
 // the DMA form; with kvx null each workgroup stages its tiles itself.  Same results.
+// cnt null with several splits: the combining launch.
 size_t fa_kvx_bytes(int n_heads, int ratio, int n_tile);
 hipError_t launch_fa_int4(float* out, const uint32_t* qq, const float* qsc, const uint32_t* kc, const float* ksc,
                           const uint32_t* vc, const float* vsc, int n_q, int n_kv, int off, int n_tile,

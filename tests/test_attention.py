@@ -517,6 +517,39 @@ def test_attention_staged_copy_matches_in_kernel_staging(rt4, torch_gpu, T, n_kv
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,n_kv,off,H,KVH,cap", [
+    (64, 3001, 2937, 2, 1, 3072),          # long enough per workgroup for one split that K/V are staged
+    (192, 6150, 5958, 3, 1, 6208),
+])
+def test_attention_long_split_staged_copy_matches_in_kernel_staging(rt4, torch_gpu, T, n_kv, off, H, KVH, cap):
+    """The same on ranges long enough (48 tiles and more a workgroup) that an eager call stages K/V."""
+    test_attention_staged_copy_matches_in_kernel_staging(rt4, torch_gpu, T, n_kv, off, H, KVH, cap)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,n_kv,H,KVH,splits", [
+    (64, 1000, 2, 1, (2, 4, 5, 8, 9, 16, 17, 40, 64)),   # combining launch; 16 tiles: empty splits above 16
+    (320, 460, 64, 8, (2, 3, 4, 5)),                     # 640+ workgroups: combined by the last split up to 4
+])
+def test_attention_split_combines(rt4, torch_gpu, T, n_kv, H, KVH, splits):
+    """Every way of combining the KV splits against one split: the same sums in another order.  Each output is a
+    ratio of sums of at most 64 tiles' fp32 terms, so it moves by less than 64 * 2^-24 * 2 of the row's magnitude."""
+    torch = torch_gpu
+    print(f"case split combines T={T} n_kv={n_kv} H={H} KVH={KVH}", flush=True)
+    rng = np.random.default_rng(31)
+    q, k, v = workload.attn_np(rng, T, n_kv, H, KVH)
+    cap = (n_kv + 63) // 64 * 64
+    g = gpu_cache(rt4, torch, q, k, v, T, cap)
+    kw = dict(n_kv=n_kv, off=n_kv - T, ratio=H // KVH)
+    one = host(rt4.attention_prefill(*g[:6], kv_splits=1, **kw))
+    for s in (0,) + splits:
+        a, b = (host(rt4.attention_prefill(*g[:6], kv_splits=s, out=torch.full((H, T, HD), float("nan"), device="cuda"),
+                                           **kw)) for _ in range(2))
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f"kv_splits={s}: repeated call differs"
+        assert rel_l2(a, one) < 64 * 2.0 ** -23, f"kv_splits={s}"
+
+
+@pytest.mark.gpu
 def test_attention_benchmark_shape_sampled(rt4, orc, torch_gpu):
     """24 heads, GQA 6:1, 1024 queries over a 32768-token cache."""
     c4 = workload.ATTN_C4
