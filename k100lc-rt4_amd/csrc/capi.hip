@@ -454,15 +454,19 @@ int rt4_gemv_w4a8(float* y, const uint32_t* wq, const uint16_t* ws, const float*
     if (rc) return rc;
     if (!aligned(wq, 16) || !aligned(y, 4) || !aligned(x, 4) || !aligned(ws, 4))
         return fail(RT4_E_ARG, "k_gemv_w4a8: misaligned pointer (wq needs 16 bytes, ws 4)");
-    rt4::GemvCfg c;
-    if ((rc = default_cfg(rows, N, K, &c))) return rc;
-    // Two launches, as the reference: the activation quantizer into library
-    // scratch, then the GEMV.  (The fused one-launch form, rt4_gemv_w4a8_cfg,
-    // re-quantizes the activations in every tile and measures slower.)
+    int cus = 0;
+    if ((rc = device_cus(&cus))) return rc;
+    const rt4::GemvCfg c = rt4::gemv_default_cfg(rows, N, K, cus);
+    // Two launches, as the reference: the activation quantizer into library scratch,
+    // then the GEMV.  One row, where it is faster: one launch that quantizes in every
+    // workgroup; it needs no scratch, which is sized all the same, so that what may be
+    // captured after a call does not depend on the form.
     hipStream_t st = as_stream(stream);
     void *q = nullptr, *s = nullptr;
     if ((rc = lib_scratch(kSlotActQ, (size_t)rows * K, &q, st))) return rc;
     if ((rc = lib_scratch(kSlotActS, (size_t)rows * (K / 128) * sizeof(float), &s, st))) return rc;
+    if (const int waves = rows == 1 ? rt4::gemv_row_waves(N, K, cus) : 0)
+        return hip_status(rt4::launch_gemv_row(y, wq, ws, x, N, K, waves, st), "k_gemv_w4a8 launch");
     hipError_t e = rt4::launch_quant_act_a8(static_cast<int8_t*>(q), static_cast<float*>(s), nullptr, x, rows, K, st);
     if (e != hipSuccess) return hip_status(e, "k_gemv_w4a8 quant launch");
     return run_gemv("k_gemv_w4a8 launch", nullptr, y, wq, ws, static_cast<const int8_t*>(q),
@@ -490,7 +494,9 @@ int rt4_gemv_w4a8_noalloc(float* y, const uint32_t* wq, const uint16_t* ws, cons
     if ((rc = noalloc_scratch(&p, st))) return rc;
     int8_t* q = reinterpret_cast<int8_t*>(p);
     float* s = reinterpret_cast<float*>(p + kNaQ);
-    // the same two launches and the same split as rt4_gemv_w4a8, so y is bit-identical
+    if (const int waves = rows == 1 ? rt4::gemv_row_waves(N, K, cus) : 0)
+        return hip_status(rt4::launch_gemv_row(y, wq, ws, x, N, K, waves, st), "rt4_gemv_w4a8_noalloc launch");
+    // the same launches and the same split as rt4_gemv_w4a8, so y is bit-identical
     hipError_t e = rt4::launch_quant_act_a8(q, s, nullptr, x, rows, K, st);
     if (e != hipSuccess) return hip_status(e, "rt4_gemv_w4a8_noalloc quant launch");
     rt4::GemvSplit sp = rt4::gemv_split(N, K, c, cus);

@@ -65,6 +65,8 @@
 // * Dot products (gemv_w4a8_dot_k, one row, K a multiple of 256 up to 8192): each
 //   wave streams two whole weight rows 1 KB per instruction and folds per group
 //   with v_dot4_i32_i8 on the vector ALU.
+// One form takes the fp32 activations of one row and is the whole linear in one launch
+// (gemv_w4a8_row_k, chosen by gemv_row_waves).
 #include "rt4_dev.h"
 #include "rt4_internal.h"
 
@@ -669,6 +671,16 @@ __global__ __launch_bounds__(512) void gemv_w4a8_tl_k(const uint32_t* __restrict
 //     to its row's fp32 partial; the wave then sums its 16 leaders per row.
 // No LDS, no cross-wave reduction and no K split; only the order of the fp32 sum
 // over groups differs from the MFMA forms.
+//
+// Sum of the 16 leaders' values (lanes 3, 7, ..., 63): within each 16-lane row by two
+// shifted adds (lane 15 of the row), then across rows by the two broadcasts (lane 63).
+__device__ __forceinline__ float dot_wave_sum(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x114, 0xF, 0xF, true));   // row_shr:4
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x118, 0xF, 0xF, true));   // row_shr:8
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xA, 0xF, false));  // row_bcast:15
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xC, 0xF, false));  // row_bcast:31
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
 template <int RPW, int NI, bool GSUM>
 __global__ __launch_bounds__(256) void gemv_w4a8_dot_k(const uint32_t* __restrict__ wq,
                                                        const uint16_t* __restrict__ ws,
@@ -738,21 +750,109 @@ __global__ __launch_bounds__(256) void gemv_w4a8_dot_k(const uint32_t* __restric
         if (RPW == 2) acc1 = fmaf((float)I, rsv[i] ? sc : 0.f, acc1);
         __builtin_amdgcn_sched_barrier(0);   // piece i's arithmetic waits for piece i's loads only
     }
-    // sum of the 16 leaders (lanes 3, 7, ..., 63) per row: within each 16-lane row by
-    // two shifted adds (lane 15 of the row), then across rows by the two broadcasts
-    // (lane 63)
-    auto wave_sum = [&](float v) __attribute__((always_inline)) {
-        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x114, 0xF, 0xF, true));   // row_shr:4
-        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x118, 0xF, 0xF, true));   // row_shr:8
-        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xA, 0xF, false));  // row_bcast:15
-        v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xC, 0xF, false));  // row_bcast:31
-        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-    };
-    const float y0 = wave_sum(acc0);
-    const float y1 = RPW == 2 ? wave_sum(acc1) : 0.f;
+    const float y0 = dot_wave_sum(acc0);
+    const float y1 = RPW == 2 ? dot_wave_sum(acc1) : 0.f;
     if (lane == 0) {
         y[n0] = y0;
         if (RPW == 2 && nrows == 2) y[n0 + 1] = y1;
+    }
+}
+
+// ---- The whole decode linear of one activation row in one launch (ROW): the dot-product
+// form with the quantizer inside.  A workgroup of W waves covers W*RPW*IT consecutive
+// weight rows.  Its threads load the fp32 row first, then every wave issues all its weight
+// loads; while those are in flight the workgroup quantizes the row into LDS (codes
+// interleaved, one fp32 scale per group: quant8_act, as quant_act_a8_k), and after one
+// barrier each wave multiplies as gemv_w4a8_dot_k does, its activations from LDS.  vmcnt
+// retires in order, so the row's loads must be the older ones.  Bound by the weight
+// stream plus the start: launch, the row's load, the quantizing and the barrier are
+// ~2 us, about what the separate quantizer launch took, and the weights arrive meanwhile
+// (gate/up 44.6 MB in 10.3 us a call, 4.5 TB/s with the launch; 11.9 with two launches).
+template <int RPW, int NI, int IT, int XI>
+__global__ __launch_bounds__(XI == 1 ? 1024 : 768) void gemv_w4a8_row_k(const uint32_t* __restrict__ wq,
+                                                        const uint16_t* __restrict__ ws,
+                                                        const float* __restrict__ xf, float* __restrict__ y, int N,
+                                                        int K, int x_aligned) {
+    static_assert(RPW == 1 || RPW == 2, "one or two rows per wave and turn");
+    constexpr int SW = (NI + 7) / 8;                  // scale dwords per lane and turn: 8 per load instruction
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, w = uniform((int)(threadIdx.x >> 6)), W = blockDim.x >> 6;
+    const int NG = K >> 7, RS = K >> 1, KB = K >> 3;
+    float* ssc = reinterpret_cast<float*>(smem + K);
+    const int n0 = uniform((int)(blockIdx.x * W + w)) * (RPW * IT);
+    // the activation row: 8 elements per lane and turn (past the row: the last 8 again;
+    // the launcher's waves and turns cover it)
+    float xv[XI][8];
+#pragma unroll
+    for (int t = 0; t < XI; t++) {
+        const int i = threadIdx.x + t * (int)blockDim.x;
+        load8(xf + 8 * (size_t)(i < KB ? i : KB - 1), x_aligned, xv[t]);
+    }
+    // the weights and their scales; a turn past the last row reads that row again
+    v4u w4[IT][NI];
+    uint32_t wsd[IT][SW];
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+        const int r0 = min(n0 + it * RPW, N - 1), nrows = min(RPW, N - r0);
+        const int span = nrows * RS, nsw = (nrows * NG) >> 1;
+        const unsigned char* wb = reinterpret_cast<const unsigned char*>(wq) + (size_t)r0 * RS;
+        const uint32_t* sb = reinterpret_cast<const uint32_t*>(ws + (size_t)r0 * NG);
+#pragma unroll
+        for (int j = 0; j < SW; j++) wsd[it][j] = sb[min(lane + 64 * j, nsw - 1)];
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int o = (i * 64 + lane) * 16;
+            w4[it][i] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(wb + (o < span ? o : span - 16)));
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < XI; t++) {
+        const int i = threadIdx.x + t * (int)blockDim.x;
+        int c[8];
+        const float s = quant8_act(xv[t], c);
+        if (i < KB) {
+            *reinterpret_cast<uint2*>(smem + 8 * (size_t)i) = interleave8(c);
+            if ((i & 15) == 0) ssc[i >> 4] = s;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; it++) {
+        const int r0 = min(n0 + it * RPW, N - 1), nrows = min(RPW, N - r0), span = nrows * RS;
+        float acc0 = 0.f, acc1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int ou = (i * 64 + lane) * 16;
+            const bool ok = ou < span;
+            const int o = ok ? ou : span - 16;
+            const int rs = RPW == 2 && o >= RS ? 1 : 0, br = o - rs * RS, gv = br >> 6;
+            const v4u x0 = *reinterpret_cast<const v4u*>(smem + 2 * br), x1 = *reinterpret_cast<const v4u*>(smem + 2 * br + 16);
+            const v4u q = w4[it][i];
+            int I = 0;
+            I = __builtin_amdgcn_sdot4((int)even_x16(q.x), (int)x0.x, I, false);
+            I = __builtin_amdgcn_sdot4((int)odd_x16(q.x), (int)x0.y, I, false);
+            I = __builtin_amdgcn_sdot4((int)even_x16(q.y), (int)x0.z, I, false);
+            I = __builtin_amdgcn_sdot4((int)odd_x16(q.y), (int)x0.w, I, false);
+            I = __builtin_amdgcn_sdot4((int)even_x16(q.z), (int)x1.x, I, false);
+            I = __builtin_amdgcn_sdot4((int)odd_x16(q.z), (int)x1.y, I, false);
+            I = __builtin_amdgcn_sdot4((int)even_x16(q.w), (int)x1.z, I, false);
+            I = __builtin_amdgcn_sdot4((int)odd_x16(q.w), (int)x1.w, I, false);
+            I += (int)dpp<0xB1>((uint32_t)I);            // quad_perm [1,0,3,2]
+            I += (int)dpp<0x4E>((uint32_t)I);            // quad_perm [2,3,0,1]
+            const int h = rs * NG + gv;                  // this piece's fp16 scale in the turn's list
+            const uint32_t pr = (uint32_t)__builtin_amdgcn_ds_bpermute((h >> 1) * 4, (int)wsd[it][i >> 3]);
+            const bool use = (lane & 3) == 3 && ok;
+            const float sc = use ? f16_bits_to_f32((uint16_t)((h & 1) ? pr >> 16 : pr & 0xFFFFu)) * 0.0625f * ssc[gv] : 0.f;
+            acc0 = fmaf((float)I, RPW == 2 && rs ? 0.f : sc, acc0);
+            if (RPW == 2) acc1 = fmaf((float)I, rs ? sc : 0.f, acc1);
+            __builtin_amdgcn_sched_barrier(0);   // piece i's arithmetic waits for piece i's loads only
+        }
+        const float y0 = dot_wave_sum(acc0), y1 = RPW == 2 ? dot_wave_sum(acc1) : 0.f;
+        if (lane == 0 && n0 + it * RPW < N) {
+            y[r0] = y0;
+            if (RPW == 2 && nrows == 2) y[r0 + 1] = y1;
+        }
     }
 }
 
@@ -773,6 +873,16 @@ hipError_t launch_dot(float* y, int32_t* gsum, const uint32_t* wq, const uint16_
 #undef RT4_DOT
         default: return hipErrorInvalidValue;
     }
+    return hipGetLastError();
+}
+
+template <int RPW, int NI, int IT, int XI>
+hipError_t launch_row(float* y, const uint32_t* wq, const uint16_t* ws, const float* xf, int N, int K, int waves,
+                      hipStream_t st) {
+    const int rows = waves * RPW * IT;
+    hipLaunchKernelGGL((gemv_w4a8_row_k<RPW, NI, IT, XI>), dim3((N + rows - 1) / rows), dim3(64 * waves),
+                       (size_t)K + (size_t)(K / kGroup) * sizeof(float), st, wq, ws, xf, y, N, K,
+                       ((uintptr_t)xf & 15) == 0);
     return hipGetLastError();
 }
 
@@ -945,6 +1055,46 @@ GemvCfg gemv_mfma_cfg(int rows, int N, int K, int cus) {
     c.waves = w < kGemvMaxWaves ? w : kGemvMaxWaves;
     c.max_split = 0;
     return c;
+}
+
+// Where the one-launch form (gemv_w4a8_row_k) takes the linear of one fp32 row, and its
+// waves per workgroup: one quantizing turn of the whole row up to K = 8192 (64 lanes x 8
+// elements a wave, rounded up to 4 waves so that they spread evenly over the SIMDs);
+// two rows a wave up to K = 6144, twice where there are many short rows.  Measured in
+// a graph (us a call, quantizer launch + GEMV -> this): K=5120 N=5120 6.58 -> 5.66,
+// N=10240 8.7 -> 7.8, N=17408 11.9 -> 10.3 (10 waves: 12.0, 8: 12.4, 16: 12.5), N=40000
+// 20.5 -> 19.9; K=2048 N=1000 4.3 -> 2.8, N=20000 7.7 -> 6.5; K=1024 N=65000 11.4 -> 9.9;
+// K=8192 N=8192 9.9 -> 8.9 (one row a wave; two 9.7), N=28672 22.7 -> 23.0, so not there.
+// Above K = 8192 every workgroup's share of the quantizing grows: K=16384 N=2048 9.95 ->
+// 7.6, K=17408 N=2560 10.1 -> 9.0 but N=5120 12.3 -> 15.6.
+int gemv_row_waves(int N, int K, int cus) {
+    const long long ncu = cus > 0 ? cus : 256;
+    if (K % 256) return 0;
+    if (K <= 8192) return (N + 15) / 16 <= 16 * ncu && (K <= 6144 || N <= 64 * ncu) ? 4 * ((K + 2047) / 2048) : 0;
+    if (K > 17408 || N > 10 * ncu) return 0;
+    return K <= 16384 ? 8 : 12;
+}
+
+hipError_t launch_gemv_row(float* y, const uint32_t* wq, const uint16_t* ws, const float* xf, int N, int K, int waves,
+                           hipStream_t st) {
+    const bool twice = K <= 4096 && N >= 8192;
+#define RT4_ROW(R, NI, IT, XI) return launch_row<R, NI, IT, XI>(y, wq, ws, xf, N, K, waves, st)
+    switch ((K + 1023) / 1024) {              // load instructions of two rows
+        case 1: if (twice) RT4_ROW(2, 1, 2, 1); RT4_ROW(2, 1, 1, 1);
+        case 2: if (twice) RT4_ROW(2, 2, 2, 1); RT4_ROW(2, 2, 1, 1);
+        case 3: if (twice) RT4_ROW(2, 3, 2, 1); RT4_ROW(2, 3, 1, 1);
+        case 4: if (twice) RT4_ROW(2, 4, 2, 1); RT4_ROW(2, 4, 1, 1);
+        case 5: RT4_ROW(2, 5, 1, 1);
+        case 6: RT4_ROW(2, 6, 1, 1);
+        case 7: case 8: RT4_ROW(1, 4, 1, 1);
+        case 9: case 10: RT4_ROW(1, 5, 1, 4);
+        case 11: case 12: RT4_ROW(1, 6, 1, 4);
+        case 13: case 14: RT4_ROW(1, 7, 1, 4);
+        case 15: case 16: RT4_ROW(1, 8, 1, 4);
+        case 17: RT4_ROW(1, 9, 1, 3);
+    }
+#undef RT4_ROW
+    return hipErrorInvalidValue;
 }
 
 bool gemv_cfg_valid(const GemvCfg& c, int K) {

@@ -12,29 +12,6 @@
 
 namespace rt4 {
 
-// Load 8 consecutive floats; vector loads when the address is 16-byte aligned.
-__device__ __forceinline__ void load8(const float* p, bool aligned, float v[8]) {
-    if (aligned) {
-        const float4 a = reinterpret_cast<const float4*>(p)[0];
-        const float4 b = reinterpret_cast<const float4*>(p)[1];
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = p[e];
-    }
-}
-
-// Eight int8 codes -> two dwords in the interleaved order [c0 c2 c4 c6 | c1 c3 c5 c7].
-__device__ __forceinline__ uint2 interleave8(const int c[8]) {
-    uint2 r;
-    r.x = (uint32_t)(c[0] & 0xFF) | (uint32_t)(c[2] & 0xFF) << 8 | (uint32_t)(c[4] & 0xFF) << 16 |
-          (uint32_t)(c[6] & 0xFF) << 24;
-    r.y = (uint32_t)(c[1] & 0xFF) | (uint32_t)(c[3] & 0xFF) << 8 | (uint32_t)(c[5] & 0xFF) << 16 |
-          (uint32_t)(c[7] & 0xFF) << 24;
-    return r;
-}
-
 // ---------------------------------------------------------------------------
 // Decode-side quantizer (restates quant_act, kernels/gemv_w4a8_core.h:34-66):
 // per (row, 128-group) s = amax>0 ? amax/127 : 1, q = clamp(lrintf(x/s), -128, 127).
@@ -57,20 +34,8 @@ __global__ __launch_bounds__(256) void quant_act_a8_k(const float* __restrict__ 
     if (i >= (K >> 3)) return;                     // K%128==0: whole 16-lane runs exit together
     float v[8];
     load8(x + (size_t)m * K + 8 * (size_t)i, ALIGNED, v);
-    float amax = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
-    amax = run_max<16>(amax);
-    const float s = amax > 0.f ? amax / 127.f : 1.f;
     int c[8];
-    if (__all(recip_div_ok(s))) {
-        const float y = 1.f / s;
-#pragma unroll
-        for (int e = 0; e < 8; e++) c[e] = clampi((int)lrintf(div_by_recip(v[e], s, y)), -128, 127);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++) c[e] = clampi((int)lrintf(v[e] / s), -128, 127);
-    }
+    const float s = quant8_act(v, c);
     *reinterpret_cast<uint2*>(xq + (size_t)m * K + 8 * (size_t)i) = interleave8(c);
     const int NG = K >> 7;
     if ((i & 15) == 0) sa[(size_t)m * NG + (i >> 4)] = s;

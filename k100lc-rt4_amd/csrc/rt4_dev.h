@@ -69,6 +69,49 @@ __device__ __forceinline__ float div_by_recip(float x, float s, float y) {
     return fmaf(fmaf(-t, s, x), y, t);
 }
 
+// Load 8 consecutive floats; vector loads when the address is 16-byte aligned.
+__device__ __forceinline__ void load8(const float* p, bool aligned, float v[8]) {
+    if (aligned) {
+        const float4 a = reinterpret_cast<const float4*>(p)[0];
+        const float4 b = reinterpret_cast<const float4*>(p)[1];
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = p[e];
+    }
+}
+
+// Eight int8 codes -> two dwords in the interleaved order [c0 c2 c4 c6 | c1 c3 c5 c7].
+__device__ __forceinline__ uint2 interleave8(const int c[8]) {
+    uint2 r;
+    r.x = (uint32_t)(c[0] & 0xFF) | (uint32_t)(c[2] & 0xFF) << 8 | (uint32_t)(c[4] & 0xFF) << 16 |
+          (uint32_t)(c[6] & 0xFF) << 24;
+    r.y = (uint32_t)(c[1] & 0xFF) | (uint32_t)(c[3] & 0xFF) << 8 | (uint32_t)(c[5] & 0xFF) << 16 |
+          (uint32_t)(c[7] & 0xFF) << 24;
+    return r;
+}
+
+// The decode quantizer on one lane's 8 elements of a 128-group, the group being an
+// aligned run of 16 lanes (all active): the scale s = amax > 0 ? amax/127 : 1 and the
+// codes clamp(lrintf(x/s), -128, 127).
+__device__ __forceinline__ float quant8_act(const float v[8], int c[8]) {
+    float amax = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
+    amax = run_max<16>(amax);
+    const float s = amax > 0.f ? amax / 127.f : 1.f;
+    if (__all(recip_div_ok(s))) {
+        const float y = 1.f / s;
+#pragma unroll
+        for (int e = 0; e < 8; e++) c[e] = clampi((int)lrintf(div_by_recip(v[e], s, y)), -128, 127);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) c[e] = clampi((int)lrintf(v[e] / s), -128, 127);
+    }
+    return s;
+}
+
 // Agent-coherent (sc1) 4-byte vector store / load of split-tile partials, each
 // with its wait in the same asm statement: the store has reached the coherent
 // level before the counter increment that publishes it, and the load's value is

@@ -62,6 +62,12 @@ hipError_t launch_gemv_w4a8(float* y, int32_t* gsum, const uint32_t* wq, const u
                             const int8_t* xq, const float* sa, const float* xf, int rows, int N, int K,
                             const GemvCfg& cfg, const GemvSplit& sp, hipStream_t st);
 
+// The decode linear of one fp32 activation row in one launch (gemv_w4a8_row_k): its waves
+// per workgroup where that form is the faster one, else 0.
+int gemv_row_waves(int N, int K, int cus);
+hipError_t launch_gemv_row(float* y, const uint32_t* wq, const uint16_t* ws, const float* xf, int N, int K, int waves,
+                           hipStream_t st);
+
 // ---- W4A4 decode GEMV (gemv4.hip): y f32 [rows][N] from RT4 weights and int4
 // activation codes aq u32 [rows][K/8] with scales sa f32 [rows][K/32].  Tiles of
 // 16 rows (rb 1), gpw 2 or 4, waves capped at the chunk count; leftover tiles cut

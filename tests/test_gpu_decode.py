@@ -131,6 +131,33 @@ def test_gemv_one_row_dot_form(rt4, orc, torch_gpu, N, K):
     assert np.array_equal(host(y).view(np.uint32), host(y2).view(np.uint32))
 
 
+@pytest.mark.parametrize("N,K", [(1, 256), (7, 512), (100, 1024), (2049, 2048), (8193, 2304), (9000, 1280), (25, 3328),
+                                 (8300, 4096), (5121, 5120), (130, 6144), (257, 6400), (77, 8192), (33, 8448),
+                                 (300, 12288), (64, 16384), (301, 16640), (2560, 17408)])
+@pytest.mark.parametrize("unaligned", [False, True])
+def test_gemv_one_row_one_launch(rt4, orc, torch_gpu, N, K, unaligned):
+    """The decode linear of one row as one launch, at the edges of its workgroup sizes, row counts and turns (its
+    rule takes all of these shapes): the codes and scales are the quantizer's, so y is the oracle's up to the order
+    of K/128 fp32 terms (K/128 * 2^-24 < 1e-5 of |y|'s terms; the bar is the GEMV's), on a fresh call and a repeat."""
+    print(f"case gemv_row N={N} K={K} unaligned={unaligned}", flush=True)
+    rng = np.random.default_rng(N + K)
+    c = workload.gemv_case(seed=5, M=1, N=N, K=K)
+    x_np = fused_edge_acts(rng, 1, K) if K >= 1024 else c["x"]
+    wq, ws = dev(torch_gpu, c["wq"]), dev(torch_gpu, c["ws"])
+    buf = torch_gpu.zeros(K + 4, dtype=torch_gpu.float32, device="cuda")
+    x = buf[1 if unaligned else 0:][:K].view(1, K)
+    x.copy_(torch_gpu.from_numpy(x_np).cuda())
+    y = rt4.gemv_w4a8(wq, ws, x, out=torch_gpu.full((1, N), float("nan"), device="cuda"))
+    y2 = rt4.gemv_w4a8(wq, ws, x)
+    yq = rt4.gemv_w4a8_q(wq, ws, *rt4.quant_act_a8(x))
+    torch_gpu.cuda.synchronize()
+    assert np.array_equal(host(y).view(np.uint32), host(y2).view(np.uint32))
+    if K <= 6144:      # two rows a wave: the terms and their order are the pre-quantized dot form's
+        assert np.array_equal(host(y).view(np.uint32), host(yq).view(np.uint32))
+    assert rel_l2(host(y), host(yq)) < TIGHT
+    assert rel_l2(host(y), orc.gemv_w4a8(c["wq"], c["ws"], x_np)) < TIGHT
+
+
 @pytest.mark.parametrize("M,N,K,gpw,waves", [(4, 300, 3072, 4, 6), (1, 17, 128, 2, 1), (2, 40, 512, 4, 1),
                                              (3, 1000, 5120, 4, 8), (4, 4176, 8192, 4, 8), (1, 520, 2944, 10, 2),
                                              (4, 64, 40960, 8, 16), (2, 48, 1920, 12, 1), (4, 33, 1408, 6, 2)])
