@@ -138,13 +138,26 @@ def release_scratch() -> None:
 
 
 # ----------------------------------------------------------- torch helpers --
+_torch_mod = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _torch_mod
+    if _torch_mod is None:
+        import torch
+        _torch_mod = torch
+    return _torch_mod
 
 
 def _stream():
-    return _P(_torch().cuda.current_stream().cuda_stream)
+    """The current stream of the current device as a hipStream_t (an int: ctypes takes
+    it for a void*).  torch.cuda.current_stream() builds a Stream object, ~2 us of a
+    call that launches ~5 us of GPU work; torch's own raw-stream query is ~0.1 us."""
+    torch = _torch()
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch._C._cuda_getDevice())
 
 
 def _ptr(t):
@@ -154,7 +167,7 @@ def _ptr(t):
         raise RT4Error("rt4_amd expects device tensors")
     if not t.is_contiguous():
         raise RT4Error("rt4_amd expects contiguous tensors")
-    return _P(t.data_ptr())
+    return t.data_ptr()
 
 
 def _empty(shape, dtype, device):
@@ -230,10 +243,9 @@ def gemv_w4a8(wq, ws, x, out=None, groups_per_wave: int = 0, waves: int = 0, k_s
     Two launches (quantizer, GEMV).  A launch configuration (see gemv_w4a8_q)
     selects rt4_gemv_w4a8_cfg instead: one launch that quantizes inside the GEMV
     (x 16-byte aligned), bit-identical output."""
-    torch = _torch()
     rows, K = x.shape
     N = wq.shape[0]
-    y = out if out is not None else _empty((rows, N), torch.float32, x.device)
+    y = out if out is not None else _empty((rows, N), _torch().float32, x.device)
     if groups_per_wave or waves or k_splits or row_blocks:
         _check(lib().rt4_gemv_w4a8_cfg(_ptr(y), _ptr(wq), _ptr(ws), _ptr(x), rows, N, K, groups_per_wave, waves,
                                        k_splits, row_blocks, _stream()))
