@@ -140,17 +140,19 @@ __device__ __forceinline__ const void* sptr(const void* p) {
 // m0 = lbase + IMM.  The scalar base keeps the per-lane address a 32-bit offset.
 // m0 is a reserved register: the compiler holds no value in it across instructions
 // and sets it right before each instruction that reads it, so these writes need
-// no clobber (declaring one is refused with a warning).
+// no clobber (declaring one is refused with a warning).  The add also writes SCC, which
+// has to be declared: the compiler schedules these between the two halves of 64-bit
+// address additions, and a carry lost there is an address 4 GiB off.
 template <int IMM>
 __device__ __forceinline__ void dma16(uint32_t voff, const void* gbase, uint32_t lbase) {
     asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sptr(gbase)),
                  "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lbase)), "n"(IMM)
-                 : "memory");
+                 : "memory", "scc");
 }
 template <int IMM>
 __device__ __forceinline__ void dma4(uint32_t voff, const void* gbase, uint32_t lbase) {
     asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sptr(gbase)),
                  "s"((uint32_t)__builtin_amdgcn_readfirstlane((int)lbase)), "n"(IMM)
-                 : "memory");
+                 : "memory", "scc");
 }
 }  // namespace rt4
