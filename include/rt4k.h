@@ -10,7 +10,7 @@
  * Library scratch: the drop-in linears' quantized activations, the split
  * workspaces of the GEMVs (W4A8 and W4A4 share one, partials plus counters that
  * every launch leaves at zero), of the GEMM and of the attention prefill, and the
- * prefill's staged K/V copy (32 KB per key tile and KV head) are one buffer per
+ * prefill's staged K/V copy (24 KB per key tile and KV head) are one buffer per
  * device and kind, grown on demand like the reference's static
  * scratch (src/k_gemv.hip:16-23).  Calls that may run at the same time on one
  * device (different streams) therefore race on it; the caller orders them, as
@@ -260,7 +260,7 @@ int rt4_kv_append_v(uint32_t* vc, float* vsc, float* stage, const float* vf, int
  * online rescaling (the running reference moves only when a tile's max exceeds
  * it by more than a factor 2^8: the same O and L, rounded differently).  Query
  * row i has position off + i.  Where each workgroup has many tiles, K/V are staged
- * once per call (codes unpacked into the MFMA operand bytes, 32 KB per key tile and
+ * once per call (codes unpacked into the MFMA operand bytes, 24 KB per key tile and
  * KV head of library scratch; at most 4 GiB), then DMA'd into LDS by the workgroups;
  * otherwise each workgroup stages its own tiles (same results).  Replaces the prefill
  * branch of k_attention (src/kernels.h:81, src/k_fa.hip:282-300; kernel fa_int4,

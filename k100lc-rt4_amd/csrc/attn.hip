@@ -19,9 +19,15 @@
 // O = O·alpha + (Σ_k P·Vcode)·(beta/7)·vsc; out = O / L.
 //
 // MI355X design.  A workgroup is 64 query rows of one head, 4 waves of 16 rows.
-// Both contractions run on v_mfma_f32_16x16x128_f8f6f4 with FP8 E4M3 operands
-// that hold the integer codes exactly, so the products come out as fp32 with no
-// int-to-float conversion:
+// Both contractions run on v_mfma_f32_16x16x128_f8f6f4 with operands that hold the
+// integer codes exactly, so the products come out as fp32 with no int-to-float
+// conversion.  There are two operand forms with the same exact products.  Tiles staged
+// once per call (below) hold FP6 E2M3 operands, code c as c/8: that instruction takes
+// 12.2 cycles where the FP8 one takes 20.2, a tile's operands are 12 KB each of K and V
+// in place of 16, and one v_cvt_scalef32_2xpk16_fp6_f32 packs a lane's 16 P codes in
+// place of eight conversions (C4 661 -> 618 us, 2048 rows over 4096 keys 163 -> 154, 1000
+// rows alone 33.5 -> 32.3).  Packing FP6 takes more instructions than FP8 does, once per
+// call but not once per workgroup, so tiles that a workgroup unpacks itself are FP8 E4M3:
 //   - K and V codes c enter as the byte c + 8 (the nibble xor 8), which is the
 //     E4M3 encoding of (c + 8)·2^-9: the subnormals 0..7 and the first normal
 //     binade 8..15 are spaced 2^-9 apart.  The offset's contribution, 8 times the
@@ -29,6 +35,7 @@
 //   - Q codes enter as their exact E4M3 values (converted once), P codes 0..7 as
 //     the subnormals p·2^-9, which v_cvt_scalef32_pk_fp8_f32 (scale 512) produces
 //     from p rounded to the nearest code.
+// FP6 codes are signed, so there is no offset to take off; ΣP is the product with ones.
 // Every partial sum is an integer times a power of two below 2^24, so each
 // MFMA result is exact.  The contractions are in transposed form so that a lane
 // always owns one query row:
@@ -46,20 +53,23 @@
 //                         two dim tiles laid out in LDS with the same key order
 //                         (one per half), so one A register block serves two
 //                         MFMAs; C = -8·ΣP·2^-18 from a fifth MFMA against
-//                         -2^-6 bytes, which also gives the row sum of P.  With
+//                         -2^-6 bytes, which also gives the row sum of P.  (FP6: the
+//                         two dim tiles' codes alternate, 32 elements a lane, and P
+//                         sits in the even or the odd ones, as its conversion leaves
+//                         it.)  With
 //                         that key order a V operand dword is exactly the even-
 //                         or odd-key bytes of one V cache dword.
 // Row max over a query's 64 keys is 15 in-lane ops plus two cross-lane steps
 // (xor 16, xor 32).  The K/V tiles reach LDS in MFMA operand order (16 bytes per
 // (subtile, group, half, lane)), so the waves only issue ds_read_b128 of ready
 // operands.  Where workgroups have many tiles (fa_plan), a pre-pass (fa_expand_kv_k)
-// unpacks every tile once per call into a copy in memory with exactly that layout, and
+// unpacks every tile once per call into a copy in memory in that order (FP6), and
 // the workgroups move each tile into LDS with global_load_lds_dwordx4 (no registers, no
 // unpacking, no LDS stores): unpacking in every workgroup repeated it once per query
 // block and split, about a tenth of the kernel at C4.  With few tiles a workgroup, or
 // without room for the copy (graph capture before the first eager call, or a copy beyond
-// 4 GiB), each workgroup stages its tiles itself from the packed cache, with the same
-// bytes.  The KV range is split over workgroups until the grid fills the CUs (fa_plan),
+// 4 GiB), each workgroup stages its tiles itself from the packed cache (FP8), with the
+// same products.  The KV range is split over workgroups until the grid fills the CUs (fa_plan),
 // down to three tiles a workgroup; a workgroup starts with one memory round trip (Q and
 // the first tiles' loads together) and converts Q by table look-up (v_perm_b32) while
 // the tiles arrive (both: C4 645 -> 639 us, 43 rows over 4096 keys 26.2 -> 25.2).
@@ -71,7 +81,7 @@
 // v_mfma_f32_16x16x1f32 (four 16x16 tiles per instruction: 2 per tile for S, 4
 // for O; four v_mfma_f32_4x4x1f32 cost about twice the matrix-core time of one),
 // and K/V are read with range-checked buffer loads.  The power-of-two factors of
-// the operand encodings (2^-9 for S, 2^-18 for O) are folded into the Q scale and
+// the operand encodings (2^-9 for S and 2^-18 for O, FP6 2^-6 for both) are folded into the Q scale and
 // the P scale, so every rounded operation is the one the integer form had.  The
 // online rescale keeps its reference until a tile max exceeds it by more than 8
 // (log2 units): the same O / L as the reference's running-max form, rounded
@@ -93,11 +103,15 @@ constexpr int NTA = 256;          // 4 waves
 constexpr float L2E = 1.4426950408889634f;
 constexpr int KU_BYTES = 4 * 4 * 64 * 16;   // unpacked K operands of one tile
 constexpr int VU_BYTES = 16 * 64 * 16;      // unpacked V operands of one tile
+constexpr int X_BYTES = 8 * 64 * 24;        // staged (FP6) K or V operands of one tile
+constexpr int X_HI = 8 * 64 * 16;           // their second plane: the last 8 of each lane's 24 bytes
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef short v2s __attribute__((ext_vector_type(2)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef unsigned v6u __attribute__((ext_vector_type(6)));
 
 // D = A·B + C on 16x16x128 FP8 E4M3 operands (format 0 for both, no block scale).
 __device__ __forceinline__ v4f mfma_e4m3(v8i a, v8i b, v4f c) {
@@ -120,6 +134,39 @@ __device__ __forceinline__ uint32_t e4m3_of_codes(uint32_t x) {
     const uint32_t ngt = __builtin_amdgcn_perm(0xB8C0C4C8u, 0xCACCCED0u, sel);   // codes -4..-1, -8..-5
     return (pos & ~m) | (ngt & m);
 }
+
+// D = A·B + C on 16x16x128 FP6 E2M3 operands (format 2 for both), six registers each.
+__device__ __forceinline__ v4f mfma_e2m3(v8i a, v8i b, v4f c) {
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 2, 2, 0, 0, 0, 0);
+}
+__device__ __forceinline__ v8i cat6(v4i lo, v2i hi) {
+    v8i r;                                       // (the last two registers are not read)
+    r[0] = lo[0], r[1] = lo[1], r[2] = lo[2], r[3] = lo[3], r[4] = hi[0], r[5] = hi[1];
+    return r;
+}
+// E2M3 codes (sign, 5-bit magnitude n = n/8 up to 15) of four int4 codes held in the low
+// nibbles of x's bytes, one per byte.
+__device__ __forceinline__ uint32_t e2m3_of_codes(uint32_t x) {
+    const uint32_t neg = (x >> 3) & 0x01010101u, m = (neg << 4) - neg;
+    return (((x & 0x0F0F0F0Fu) ^ m) + neg) | (neg << 5);
+}
+// Four 6-bit codes (one per byte) side by side in 24 bits.
+__device__ __forceinline__ uint32_t pack24(uint32_t x) {
+    return (x & 0x3Fu) | ((x >> 2) & 0xFC0u) | ((x >> 4) & 0x3F000u) | ((x >> 6) & 0xFC0000u);
+}
+// The E2M3 operand of 32 codes in four dwords w: per dword the even, then the odd nibbles.
+__device__ __forceinline__ void e2m3_operand(const uint32_t (&w)[4], uint32_t (&o)[6]) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const uint32_t t0 = pack24(e2m3_of_codes(w[2 * h])), t1 = pack24(e2m3_of_codes(w[2 * h] >> 4));
+        const uint32_t t2 = pack24(e2m3_of_codes(w[2 * h + 1])), t3 = pack24(e2m3_of_codes(w[2 * h + 1] >> 4));
+        o[3 * h] = t0 | t1 << 24;
+        o[3 * h + 1] = t1 >> 8 | t2 << 16;
+        o[3 * h + 2] = t2 >> 16 | t3 << 8;
+    }
+}
+// max that returns NaN if an operand is one (fmaxf drops it).
+__device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 
 // Key order within a 16-key subtile: output register r of lane group G holds key
 // key_of_slot(G, r); the K row fed to the MFMA at slot 4G + r is that key.
@@ -144,7 +191,7 @@ constexpr int kRsrcW3 = 0x00020000;    // dword 3 of a buffer resource: 32-bit d
 
 // The staged form of a 64-key tile: the MFMA operand bytes in the order the waves
 // read them, 16 KB for K and 16 KB for V.  These write one thread's share of a
-// tile's block (in LDS, or its copy in memory for the DMA path).
+// tile's block in LDS (put_k6 and put_v6 below: of its copy in memory).
 //
 // K: key kk = tid % 64, dims 64p .. 64p + 63 (p = tid / 64, code dwords j = 0..7,
 // k0 then k1): group p/2, lane group G' = 2(p%2) + j/4 of the operand, half (j/2)%2
@@ -182,6 +229,52 @@ __device__ __forceinline__ void put_v_slots(unsigned char* blk, const uint32_t (
     }
 }
 
+// The same for the staged copy: FP6 operands, 24 bytes per lane in two planes (16 and 8
+// bytes), piece p of a block at 64 lanes each.
+// K: piece (subtile, group); a lane's 32 elements are its 32 dims in e2m3_operand's order.
+__device__ __forceinline__ void put_k6(unsigned char* blk, v4u k0, v4u k1, int tid) {
+    const int kk = tid & 63, p = tid >> 6;
+    const uint32_t d[2][4] = {{k0.x, k0.y, k0.z, k0.w}, {k1.x, k1.y, k1.z, k1.w}};
+#pragma unroll
+    for (int h = 0; h < 2; h++) {                // lane group 2 (p % 2) + h of the operand
+        uint32_t o[6];
+        e2m3_operand(d[h], o);
+        const int at = ((kk >> 4) * 2 + (p >> 1)) * 64 + 16 * (2 * (p & 1) + h) + slot_of_key(kk & 15);
+        *reinterpret_cast<uint4*>(blk + at * 16) = make_uint4(o[0], o[1], o[2], o[3]);
+        *reinterpret_cast<uint2*>(blk + X_HI + at * 8) = make_uint2(o[4], o[5]);
+    }
+}
+// V: piece j holds dim tiles 2j (even elements) and 2j + 1 (odd ones); element pair i of
+// lane group G is key 16 (i/4) + key_of_slot(G, i % 4), as P holds them.  A thread makes
+// its dim's 16 codes of each group, 12 bits apart; the thread of the other tile (lane
+// xor 16) supplies the fields between.
+__device__ __forceinline__ void put_v6(unsigned char* blk, const uint32_t (&vw)[8], int tid) {
+    const int dt = tid >> 4, odd = dt & 1;
+#pragma unroll
+    for (int G = 0; G < 4; G++) {
+        uint32_t o[6];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            // 8 codes: bytes of X (subtile 2h) and Y (2h + 1)
+            const uint32_t a = vw[4 * h + (G >> 1)], b = vw[4 * h + 2 + (G >> 1)];
+            const uint32_t X = e2m3_of_codes((G & 1) ? a >> 4 : a), Y = e2m3_of_codes((G & 1) ? b >> 4 : b);
+            const uint32_t w0 = (X & 0x3Fu) | (X & 0x3F00u) << 4 | (X & 0x3F0000u) << 8;
+            const uint32_t w1 = ((X >> 20) & 0x3F0u) | (Y & 0x3Fu) << 16 | (Y & 0x3F00u) << 20;
+            const uint32_t w2 = ((Y >> 12) & 3u) | (Y & 0x3F0000u) >> 8 | ((Y >> 4) & 0x03F00000u);
+            o[3 * h] = odd ? w0 << 6 : w0;
+            o[3 * h + 1] = odd ? w1 << 6 | w0 >> 26 : w1;
+            o[3 * h + 2] = odd ? w2 << 6 | w1 >> 26 : w2;
+        }
+#pragma unroll
+        for (int i = 0; i < 6; i++) o[i] |= (uint32_t)__shfl_xor((int)o[i], 16);
+        if ((G & 1) == odd) {                    // the two threads write two groups each
+            const int at = (dt >> 1) * 64 + G * 16 + (tid & 15);
+            *reinterpret_cast<uint4*>(blk + at * 16) = make_uint4(o[0], o[1], o[2], o[3]);
+            *reinterpret_cast<uint2*>(blk + X_HI + at * 8) = make_uint2(o[4], o[5]);
+        }
+    }
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------- prefill --
@@ -198,8 +291,10 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
                                                     float2* __restrict__ mlpart, int* __restrict__ cnt,
                                                     const unsigned char* __restrict__ kx,
                                                     const unsigned char* __restrict__ vx) {
-    __shared__ __align__(16) unsigned char ku[2 * KU_BYTES];   // x2: [subtile][k-step][lane] x 16 B
-    __shared__ __align__(16) unsigned char vu[2 * VU_BYTES];   // x2: [dim tile][lane] x 16 B
+    // DMA: the staged FP6 operands; otherwise FP8 ones unpacked here
+    constexpr int KB = DMA ? X_BYTES : KU_BYTES, VB = DMA ? X_BYTES : VU_BYTES;
+    __shared__ __align__(16) unsigned char ku[2 * KB];   // x2: [piece][lane] x 16 B (DMA: then x 8 B)
+    __shared__ __align__(16) unsigned char vu[2 * VB];
     __shared__ __align__(16) float ks_l[2][2 * BNK];
     __shared__ __align__(16) float vs_l[2][HD];
     __shared__ int s_last;
@@ -245,6 +340,12 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
 #pragma unroll
         for (int g = 0; g < 2; g++) {
             const uint32_t w[4] = {qraw[g].x, qraw[g].y, qraw[g].z, qraw[g].w};
+            if constexpr (DMA) {
+                uint32_t o[6];
+                e2m3_operand(w, o);
+                qop[g] = cat6(v4i{(int)o[0], (int)o[1], (int)o[2], (int)o[3]}, v2i{(int)o[4], (int)o[5]});
+                continue;
+            }
 #pragma unroll
             for (int m = 0; m < 4; m++) {
                 qs[g] = __builtin_amdgcn_sdot8((int)w[m], 0x11111111, qs[g], false);
@@ -254,11 +355,14 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
             qs[g] += __shfl_xor(qs[g], 16);
             qs[g] += __shfl_xor(qs[g], 32);
         }
+        // (DMA: qs is 0 and unused, the FP6 codes carry no offset)
         const float c0 = (float)(-8 * qs[0]) * (1.f / 512.f), c1 = (float)(-8 * qs[1]) * (1.f / 512.f);
         cS0 = v4f{c0, c0, c0, c0};
         cS1 = v4f{c1, c1, c1, c1};
     };
-    // S in log2 units: log2(e) and the 2^9 of the offset K operand go into the Q scales
+    // S in log2 units: log2(e) and the power of two of the operand encodings (2^-9 of the
+    // FP8 K operand, 2^-6 of FP6 K and Q) go into the Q scales
+    constexpr float QSCALE = DMA ? 64.f : 512.f;
     float A0 = qsc[qrow], A1 = qsc[n_q + qrow];
 
     float O[16][4];
@@ -332,37 +436,29 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
     auto store_k = [&](const StageK& S, int b, int t) {
         // codes (unless DMA brings them) and scales; keys >= n_kv read as zero codes
         // (flash_attn_core.h:143-147), i.e. bytes 8
-        if constexpr (!DMA) put_k_slots(ku + b * KU_BYTES, S.k0, S.k1, tid);
+        if constexpr (!DMA) put_k_slots(ku + b * KB, S.k0, S.k1, tid);
         if (tid < 2 * BNK) ks_l[b][tid] = t * BNK + (tid & 63) < kv_cap ? S.ks : 1.f;
     };
     auto store_v = [&](const StageV& S, int b, int t) {
         // a group of 8 keys is read only if it is whole (flash_attn_core.h:150-152),
         // else zero codes
-        if constexpr (!DMA) put_v_slots(vu + b * VU_BYTES, S.v, tid);
+        if constexpr (!DMA) put_v_slots(vu + b * VB, S.v, tid);
         vs_l[b][tid] = t < kv_cap / BNK ? S.vs : 1.f;
     };
     // DMA path: tiles t of K and V as staged blocks from the expanded copy (kx, vx:
-    // [KV head][tile][16 KB]) straight into LDS buffers bk / bv, one 1 KB piece per
-    // instruction, four per wave.  Tiles past the last one (the prefetch runs ahead)
+    // [KV head][tile][12 KB]) straight into LDS buffers bk / bv, one 1 KB piece per
+    // instruction, three per wave.  Tiles past the last one (the prefetch runs ahead)
     // read the last tile instead, into buffers nobody reads.
-    auto dma_k = [&](int t, int b) {
+    auto dma_x = [&](const unsigned char* x, unsigned char* buf, int t) {
         t = t < n_tile - 1 ? t : n_tile - 1;
-        const unsigned char* src = kx + ((size_t)vh * n_tile + t) * KU_BYTES;
-        const uint32_t dst = lds_addr(ku) + b * KU_BYTES + 4 * w * 1024;
-        dma16<0>(lane * 16 + 4 * w * 1024, src, dst);
-        dma16<1024>(lane * 16 + (4 * w + 1) * 1024, src, dst);
-        dma16<2048>(lane * 16 + (4 * w + 2) * 1024, src, dst);
-        dma16<3072>(lane * 16 + (4 * w + 3) * 1024, src, dst);
+        const unsigned char* src = x + ((size_t)vh * n_tile + t) * X_BYTES;
+        const uint32_t dst = lds_addr(buf) + 3 * w * 1024;
+        dma16<0>(lane * 16 + 3 * w * 1024, src, dst);
+        dma16<1024>(lane * 16 + (3 * w + 1) * 1024, src, dst);
+        dma16<2048>(lane * 16 + (3 * w + 2) * 1024, src, dst);
     };
-    auto dma_v = [&](int t, int b) {
-        t = t < n_tile - 1 ? t : n_tile - 1;
-        const unsigned char* src = vx + ((size_t)vh * n_tile + t) * VU_BYTES;
-        const uint32_t dst = lds_addr(vu) + b * VU_BYTES + 4 * w * 1024;
-        dma16<0>(lane * 16 + 4 * w * 1024, src, dst);
-        dma16<1024>(lane * 16 + (4 * w + 1) * 1024, src, dst);
-        dma16<2048>(lane * 16 + (4 * w + 2) * 1024, src, dst);
-        dma16<3072>(lane * 16 + (4 * w + 3) * 1024, src, dst);
-    };
+    auto dma_k = [&](int t, int b) { dma_x(kx, ku + b * KB, t); };
+    auto dma_v = [&](int t, int b) { dma_x(vx, vu + b * VB, t); };
 
     // front of tile t (K in buffer b): S^T = K Q^T for the 4 subtiles of 16 keys,
     // the causal mask (MASK: the tile may reach past a row of this workgroup), the
@@ -375,7 +471,7 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
     auto front = [&](int t, int b, auto mask_tag) -> Front {
         constexpr bool MASK = decltype(mask_tag)::value;
         const int kb = t * BNK;
-        const unsigned char* kub = ku + b * KU_BYTES;
+        const unsigned char* kub = ku + b * KB;
         const float* ksb = ks_l[b];
         float sv[4][4];
         // key scale x query scale of every entry (subtile kt in registers 4kt..4kt+3)
@@ -383,10 +479,19 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
         const v16f c1 = outer16(ksb[BNK + kslot], A1);
 #pragma unroll
         for (int kt = 0; kt < 4; kt++) {
-            // pieces (kt, group, half) at ((kt * 2 + group) * 2 + half) * 64
-            const v4i* kp = reinterpret_cast<const v4i*>(kub) + (kt * 4) * 64 + lane;
-            const v4f a0 = mfma_e4m3(cat8(kp[0], kp[64]), qop[0], cS0);
-            const v4f a1 = mfma_e4m3(cat8(kp[128], kp[192]), qop[1], cS1);
+            v4f a0, a1;
+            if constexpr (DMA) {
+                // pieces (kt, group) at (kt * 2 + group) * 64, in two planes
+                const v4i* kp = reinterpret_cast<const v4i*>(kub) + (kt * 2) * 64 + lane;
+                const v2i* kh = reinterpret_cast<const v2i*>(kub + X_HI) + (kt * 2) * 64 + lane;
+                a0 = mfma_e2m3(cat6(kp[0], kh[0]), qop[0], v4f{0.f, 0.f, 0.f, 0.f});
+                a1 = mfma_e2m3(cat6(kp[64], kh[64]), qop[1], v4f{0.f, 0.f, 0.f, 0.f});
+            } else {
+                // pieces (kt, group, half) at ((kt * 2 + group) * 2 + half) * 64
+                const v4i* kp = reinterpret_cast<const v4i*>(kub) + (kt * 4) * 64 + lane;
+                a0 = mfma_e4m3(cat8(kp[0], kp[64]), qop[0], cS0);
+                a1 = mfma_e4m3(cat8(kp[128], kp[192]), qop[1], cS1);
+            }
 #pragma unroll
             for (int r = 0; r < 4; r++) sv[kt][r] = fmaf(a1[r], c1[4 * kt + r], a0[r] * c0[4 * kt + r]);
         }
@@ -404,12 +509,14 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
 #pragma unroll
         for (int kt = 0; kt < 4; kt++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) m = fmaxf(m, sv[kt][r]);
+            for (int r = 0; r < 4; r++) m = DMA ? max_nan(m, sv[kt][r]) : fmaxf(m, sv[kt][r]);
         {   // xor 16 and xor 32 partners: each swap leaves a lane its value and its partner's
             const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-            m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+            m = DMA ? max_nan(__uint_as_float(a[0]), __uint_as_float(a[1]))
+                    : fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
             const auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-            m = fmaxf(__uint_as_float(c[0]), __uint_as_float(c[1]));
+            m = DMA ? max_nan(__uint_as_float(c[0]), __uint_as_float(c[1]))
+                    : fmaxf(__uint_as_float(c[0]), __uint_as_float(c[1]));
         }
         // Fully masked row in this tile: take the running reference (the state after
         // the previous tile), so nothing is rescaled and every P is 2^(-inf) = 0.  (The
@@ -429,6 +536,34 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
         // its operands), so S - m <= 0 and p <= 7 (1 + a few ulp) < 7.5; a fully
         // masked row has m = rref, S - m = -inf and P = 0.
         const float m7 = m - 2.807354922057604f;   // m - log2(7)
+        Front f;
+        f.m = m;
+        if constexpr (DMA) {
+            // One instruction turns 2 x 16 values into 32 E2M3 codes, the two inputs taking
+            // turns: p/8 rounded to nearest (ties to even) is code p's own encoding.  P in
+            // every pair of elements, masked to the even ones (dim tiles 2j) and to the odd
+            // ones (2j + 1).  FP6 has no NaN: a NaN among the S makes m one (above), and
+            // through it beta, so the row comes out NaN as it does with FP8 operands.
+            v16f pv;
+#pragma unroll
+            for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) pv[4 * kt + r] = __builtin_amdgcn_exp2f(sv[kt][r] - m7);
+            v6u pp = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(pv, pv, 8.f);
+            // The conversion writes its result over several passes, but the compiler does not
+            // keep that result off the sources: the inputs live on past it, so it has to.
+            asm volatile("" : "+v"(pp) : "v"(pv));
+            constexpr uint32_t even[3] = {0x3F03F03Fu, 0xF03F03F0u, 0x03F03F03u};
+            const v4i lo = {(int)(pp[0] & even[0]), (int)(pp[1] & even[1]), (int)(pp[2] & even[2]), (int)(pp[3] & even[0])};
+            const v4i hi = {(int)(pp[0] & ~even[0]), (int)(pp[1] & ~even[1]), (int)(pp[2] & ~even[2]), (int)(pp[3] & ~even[0])};
+            f.p_lo = cat6(lo, v2i{(int)(pp[4] & even[1]), (int)(pp[5] & even[2])});
+            f.p_hi = cat6(hi, v2i{(int)(pp[4] & ~even[1]), (int)(pp[5] & ~even[2])});
+            // ΣP/8 of the row over the tile's 64 keys: A elements 1.0 (code 8)
+            const v8i ones = cat6(v4i{0x08208208, (int)0x82082082u, 0x20820820, 0x08208208},
+                                  v2i{(int)0x82082082u, 0x20820820});
+            f.corr = mfma_e2m3(ones, f.p_lo, v4f{0.f, 0.f, 0.f, 0.f});
+            return f;
+        }
         uint32_t pk[4];
 #pragma unroll
         for (int kt = 0; kt < 4; kt++) {
@@ -443,10 +578,8 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
             w = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(w, p[2], p[3], 512.f, true);
             pk[kt] = __builtin_bit_cast(uint32_t, w);
         }
-        Front f;
         f.p_lo = v8i{(int)pk[0], (int)pk[1], (int)pk[2], (int)pk[3], 0, 0, 0, 0};
         f.p_hi = v8i{0, 0, 0, 0, (int)pk[0], (int)pk[1], (int)pk[2], (int)pk[3]};
-        f.m = m;
         // -8·Σ_k P·2^-18 of the row over the tile's 64 keys on the matrix pipe: A
         // bytes -2^-6 (E4M3 0x88) against the P bytes give it in every output row.
         // Two chained 16x16x32 FP8 MFMAs over the code dwords as they are (a lane's
@@ -470,7 +603,7 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
     // reference's (flash_attn_core.h, running max), so O / L and the split combine
     // (which rescales by the stored rref) are the same quantities, rounded
     // differently; the rescale of O (64 multiplies) runs a few times per split
-    // instead of on about a third of the tiles (configs[4] 802 -> 764 us).  With
+    // instead of on about a third of the tiles (C4 802 -> 764 us).  With
     // beta <= 2^8, O stays finite for V scales below about 10^28.
     auto update = [&](const Front& f) -> float {
         if (__any(f.m > rref + 8.f)) {      // a wave-uniform branch
@@ -487,8 +620,9 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
         }
         const float beta = __builtin_amdgcn_exp2f(f.m - rref);
         const float pb = beta * (1.f / 7.f);
-        L += (f.corr[0] * -32768.f) * pb;     // corr * -2^15 = ΣP exactly
-        return pb * 262144.f;
+        // corr is ΣP/8 (FP6) or -8·ΣP·2^-18: ΣP exactly; the PV operand bytes carry 2^-6 or 2^-18
+        L += (f.corr[0] * (DMA ? 8.f : -32768.f)) * pb;
+        return pb * (DMA ? 64.f : 262144.f);
     };
     // back: O^T += (V^T P^T) * vsc * pbv per dim tile, V in buffer b.  One A
     // register block holds the V operands of dim tiles 2j and 2j + 1 (halves 0 and
@@ -497,34 +631,65 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
     // dim tiles are read while the current four are multiplied and folded (left to
     // itself the compiler reads each pair just before its MFMAs and waits for it).
     auto back = [&](const v8i p_lo, const v8i p_hi, const v4f cc, float pbv, int b) {
-        const unsigned char* vub = vu + b * VU_BYTES;
+        const unsigned char* vub = vu + b * VB;
         const float* vsb = vs_l[b];
         // raised issue priority over the PV block: the other wave on the SIMD then
-        // fills the matrix-core gaps with its S/P work (configs[4] 830 -> 816 us)
+        // fills the matrix-core gaps with its S/P work (C4 830 -> 816 us)
         __builtin_amdgcn_s_setprio(1);
-        v4i vn[4];
+        if constexpr (DMA) {
+            const v4i* vp = reinterpret_cast<const v4i*>(vub) + lane;
+            const v2i* vq = reinterpret_cast<const v2i*>(vub + X_HI) + lane;
+            const v4f z = {0.f, 0.f, 0.f, 0.f};
+            v4i vn[2] = {vp[0], vp[64]};
+            v2i wn[2] = {vq[0], vq[64]};
 #pragma unroll
-        for (int d4 = 0; d4 < 4; d4++) vn[d4] = *(reinterpret_cast<const v4i*>(vub) + d4 * 64 + lane);
+            for (int dq = 0; dq < 4; dq++) {
+                const v8i a[2] = {cat6(vn[0], wn[0]), cat6(vn[1], wn[1])};
+                if (dq < 3) {
 #pragma unroll
-        for (int dq = 0; dq < 4; dq++) {
-            v4i vcur[4];
+                    for (int d = 0; d < 2; d++) {
+                        vn[d] = vp[(2 * dq + 2 + d) * 64];
+                        wn[d] = vq[(2 * dq + 2 + d) * 64];
+                    }
+                }
+                const v16f ps = outer16(vsb[64 * dq + lane], pbv);   // vsc * pbv of dim tiles 4dq..4dq+3
 #pragma unroll
-            for (int d4 = 0; d4 < 4; d4++) vcur[d4] = vn[d4];
-            if (dq < 3) {
+                for (int d = 0; d < 2; d++) {
+                    const v4f acc0 = mfma_e2m3(a[d], p_lo, z);
+                    const v4f acc1 = mfma_e2m3(a[d], p_hi, z);
+                    const int dt = 4 * dq + 2 * d;
 #pragma unroll
-                for (int d4 = 0; d4 < 4; d4++) vn[d4] = *(reinterpret_cast<const v4i*>(vub) + (4 * dq + 4 + d4) * 64 + lane);
+                    for (int r = 0; r < 4; r++) {
+                        O[dt][r] = fmaf(acc0[r], ps[8 * d + r], O[dt][r]);
+                        O[dt + 1][r] = fmaf(acc1[r], ps[8 * d + 4 + r], O[dt + 1][r]);
+                    }
+                }
             }
-            const v16f ps = outer16(vsb[64 * dq + lane], pbv);   // vsc * pbv of dim tiles 4dq..4dq+3
+        } else {
+            v4i vn[4];
 #pragma unroll
-            for (int d2 = 0; d2 < 4; d2 += 2) {
-                const v8i a = cat8(vcur[d2], vcur[d2 + 1]);
-                const v4f acc0 = mfma_e4m3(a, p_lo, cc);
-                const v4f acc1 = mfma_e4m3(a, p_hi, cc);
-                const int dt = 4 * dq + d2;
+            for (int d4 = 0; d4 < 4; d4++) vn[d4] = *(reinterpret_cast<const v4i*>(vub) + d4 * 64 + lane);
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    O[dt][r] = fmaf(acc0[r], ps[4 * d2 + r], O[dt][r]);
-                    O[dt + 1][r] = fmaf(acc1[r], ps[4 * d2 + 4 + r], O[dt + 1][r]);
+            for (int dq = 0; dq < 4; dq++) {
+                v4i vcur[4];
+#pragma unroll
+                for (int d4 = 0; d4 < 4; d4++) vcur[d4] = vn[d4];
+                if (dq < 3) {
+#pragma unroll
+                    for (int d4 = 0; d4 < 4; d4++) vn[d4] = *(reinterpret_cast<const v4i*>(vub) + (4 * dq + 4 + d4) * 64 + lane);
+                }
+                const v16f ps = outer16(vsb[64 * dq + lane], pbv);   // vsc * pbv of dim tiles 4dq..4dq+3
+#pragma unroll
+                for (int d2 = 0; d2 < 4; d2 += 2) {
+                    const v8i a = cat8(vcur[d2], vcur[d2 + 1]);
+                    const v4f acc0 = mfma_e4m3(a, p_lo, cc);
+                    const v4f acc1 = mfma_e4m3(a, p_hi, cc);
+                    const int dt = 4 * dq + d2;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        O[dt][r] = fmaf(acc0[r], ps[4 * d2 + r], O[dt][r]);
+                        O[dt + 1][r] = fmaf(acc1[r], ps[4 * d2 + 4 + r], O[dt + 1][r]);
+                    }
                 }
             }
         }
@@ -549,8 +714,8 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
         load_k(sk1, t0 + 1);
         asm volatile("" ::: "memory");
         make_q();
-        A0 *= L2E * 512.f;
-        A1 *= L2E * 512.f;
+        A0 *= L2E * QSCALE;
+        A1 *= L2E * QSCALE;
         store_k(sk, t0 & 1, t0);
         store_v(sv, t0 & 1, t0);
         store_k(sk1, (t0 + 1) & 1, t0 + 1);
@@ -747,17 +912,16 @@ __global__ __launch_bounds__(256) void fa_combine_k(const float* __restrict__ op
         make_float2(l > 0.f ? acc.x / l : 0.f, l > 0.f ? acc.y / l : 0.f);
 }
 
-// Staged K/V blocks of every tile of every KV head, for the DMA path: the kernel's
-// own staging (same loads, range checks and byte layout), run once per call instead
-// of once per query block and split.  Block (vh, t) of kx / vx holds the 16 KB that
-// tile t's staging writes to LDS.
+// Staged K/V blocks of every tile of every KV head, for the DMA path, made once per call
+// instead of once per query block and split (same loads and range checks as the kernel's
+// own staging).  Block (vh, t) of kx / vx holds the 12 KB of FP6 operands of tile t.
 __global__ __launch_bounds__(256) void fa_expand_kv_k(const uint32_t* __restrict__ kc,
                                                       const uint32_t* __restrict__ vc,
                                                       unsigned char* __restrict__ kx,
                                                       unsigned char* __restrict__ vx, int n_kv, int n_tile,
                                                       int kv_cap) {
     const int t = blockIdx.x, vh = blockIdx.y, tid = threadIdx.x;
-    const size_t blk = ((size_t)vh * n_tile + t) * KU_BYTES;
+    const size_t blk = ((size_t)vh * n_tile + t) * X_BYTES;
     if (blockIdx.z == 0) {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint32_t*>(kc + (size_t)vh * kv_cap * KDW), 0, n_kv * KDW * 4, kRsrcW3);
@@ -765,7 +929,7 @@ __global__ __launch_bounds__(256) void fa_expand_kv_k(const uint32_t* __restrict
         const int sk = (int)((uint32_t)t * (uint32_t)(BNK * KDW * 4));
         const v4u k0 = __builtin_amdgcn_raw_buffer_load_b128(rs, off, sk, 0);
         const v4u k1 = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16, sk, 0);
-        put_k_slots(kx + blk, k0, k1, tid);
+        put_k6(kx + blk, k0, k1, tid);
     } else {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint32_t*>(vc + (size_t)vh * (kv_cap / 8) * HD), 0, (n_kv / 8) * HD * 4, kRsrcW3);
@@ -774,7 +938,7 @@ __global__ __launch_bounds__(256) void fa_expand_kv_k(const uint32_t* __restrict
 #pragma unroll
         for (int g = 0; g < 8; g++)
             vw[g] = __builtin_amdgcn_raw_buffer_load_b32(rs, tid * 4 + (g & 3) * HD * 4, sv + (g >> 2) * 4 * HD * 4, 0);
-        put_v_slots(vx + blk, vw, tid);
+        put_v6(vx + blk, vw, tid);
     }
 }
 
@@ -813,12 +977,15 @@ FaPlan fa_plan(int n_q, int n_heads, int ratio, int off, int n_tile, int cus, in
         p.nsplit = kv_splits;
         p.inline_combine = kv_splits <= kFaInlineSplits && (long long)items * kv_splits > slots;
     }
-    // Stage K/V once for all (a launch, ~4 us and 6.5 ns a tile and KV head), or in every
-    // workgroup, which costs it 0.2 us a tile (0.4 where two share a CU): 43 rows over 4096
-    // keys 29 us staged, 25 not; C4 639 staged, 758 not.
+    // Stage K/V once for all (a launch, ~4 us and 5.5 ns a tile and KV head), or in every
+    // workgroup, which costs it 0.3 us a tile (0.45 where two share a CU), the FP8 form's
+    // slower products included.  Measured (us, 24 heads over 4 unless noted, staged / not): 43
+    // rows over 4096 keys 26.6 / 22.4, 128 over 16384 62.3 / 65.4, 256 over 2048 35.6 / 36.0,
+    // 1000 rows alone 32.3 / 33.6, 512 alone 19.8 / 19.4, 64 over 32768 with 8 heads over 8
+    // 60.9 / 36.3, C4 618 / 756.
     const long long blocks = (long long)items * p.nsplit;
     const double visits = (double)((nt + p.nsplit - 1) / p.nsplit) * (double)((blocks + slots - 1) / slots);
-    p.staged = visits * (blocks <= cus ? 0.2 : 0.4) > 4.0 + 0.0065 * (double)n_tile * (n_heads / ratio);
+    p.staged = visits * (blocks <= cus ? 0.3 : 0.45) > 4.0 + 0.0055 * (double)n_tile * (n_heads / ratio);
     return p;
 }
 
@@ -831,7 +998,7 @@ size_t fa_cnt_bytes(int n_q, int n_heads, int nsplit) {
 }
 
 size_t fa_kvx_bytes(int n_heads, int ratio, int n_tile) {
-    return (size_t)2 * (size_t)(n_heads / ratio) * (size_t)n_tile * KU_BYTES;
+    return (size_t)2 * (size_t)(n_heads / ratio) * (size_t)n_tile * X_BYTES;
 }
 
 hipError_t launch_fa_int4(float* out, const uint32_t* qq, const float* qsc, const uint32_t* kc, const float* ksc,
@@ -848,7 +1015,7 @@ hipError_t launch_fa_int4(float* out, const uint32_t* qq, const float* qsc, cons
     } else {
         const int kvh = n_heads / ratio;
         unsigned char* kx = static_cast<unsigned char*>(kvx);
-        unsigned char* vx = kx + (size_t)kvh * n_tile * KU_BYTES;
+        unsigned char* vx = kx + (size_t)kvh * n_tile * X_BYTES;
         hipLaunchKernelGGL(fa_expand_kv_k, dim3(n_tile, kvh, 2), dim3(256), 0, st, kc, vc, kx, vx, n_kv, n_tile, kv_cap);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         hipLaunchKernelGGL(fa_int4_k<true>, grid, dim3(NTA), 0, st, qq, qsc, kc, ksc, vc, vsc, out, n_q, n_kv, off,

@@ -699,7 +699,7 @@ int rt4_kv_append_v(uint32_t* vc, float* vsc, float* stage, const float* vf, int
 // The prefill kernel addresses one KV head's cache through 32-bit buffer offsets
 // (kv_cap * 128 bytes of K codes, plus up to three tiles read past the end).
 constexpr int kMaxKvCap = (1 << 24) - 64;
-// Largest staged K/V copy the prefill allocates (4 GiB: 65536 tiles x KV heads).
+// Largest staged K/V copy the prefill allocates (4 GiB: 174762 tiles x KV heads).
 constexpr size_t kMaxKvxBytes = (size_t)4 << 30;
 
 int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, const uint32_t* kc,

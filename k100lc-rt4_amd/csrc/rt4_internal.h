@@ -124,7 +124,7 @@ struct FaPlan {
 FaPlan fa_plan(int n_q, int n_heads, int ratio, int off, int n_tile, int cus, int kv_splits);
 size_t fa_part_bytes(int n_q, int n_heads, int nsplit);
 size_t fa_cnt_bytes(int n_q, int n_heads, int nsplit);
-// Bytes of the staged K/V copy the DMA form of the prefill reads (two 16 KB blocks
+// Bytes of the staged K/V copy the DMA form of the prefill reads (two 12 KB blocks
 // per tile and KV head).  launch_fa_int4 with kvx (that many bytes) fills it and runs
 // the DMA form; with kvx null each workgroup stages its tiles itself.  Same results.
 // cnt null with several splits: the combining launch.

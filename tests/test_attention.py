@@ -527,6 +527,43 @@ def test_attention_long_split_staged_copy_matches_in_kernel_staging(rt4, torch_g
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("odd", [False, True])
+def test_attention_staged_operands_of_every_code(rt4, torch_gpu, odd):
+    """The staged copy holds other operand encodings than the workgroups' own staging (6-bit against 8-bit floats).
+    Both hold every code exactly (-8 too, which the appends never write), so caches of random nibbles give the same
+    bits; with NaN and infinite scales (odd) the same elements are NaN and the others keep their bits."""
+    torch = torch_gpu
+    T, n_kv, H, KVH, cap = 192, 6150, 3, 1, 6208
+    off = n_kv - T
+    print(f"case staged operands of every code T={T} n_kv={n_kv} odd={odd}", flush=True)
+    rng = np.random.default_rng(37)
+    words = lambda *n: dev(torch, rng.integers(0, 2 ** 32, n, dtype=np.uint64).astype(np.uint32).view(np.int32))
+    scales = lambda lo, *n: dev(torch, (lo * (1 + rng.random(n))).astype(np.float32))
+    qq, kc, vc = words(H, T, 32), words(KVH, cap, 32), words(KVH, cap // 8, HD)
+    qs, ksc, vsc = scales(0.05, H, 2, T), scales(0.05, KVH, 2, cap), scales(0.1, KVH, cap // BN, HD)
+    if odd:
+        qs[0, 0, 5], qs[1, 1, 70], qs[2, 0, 9] = float("nan"), float("inf"), 0.0
+        ksc[0, 0, off + 150], ksc[0, 1, off + 100] = float("nan"), float("inf")
+        vsc[0, 3, 17], vsc[0, 90, 200] = float("nan"), float("inf")
+    g, kw = (qq, qs, kc, ksc, vc, vsc), dict(n_kv=n_kv, off=off, ratio=H // KVH, kv_splits=1)
+    staged = host(rt4.attention_prefill(*g, **kw))
+    torch.cuda.synchronize()
+    rt4.release_scratch()
+    out = torch.full((H, T, HD), float("nan"), dtype=torch.float32, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):                  # no room for the copy: each workgroup stages its tiles
+        rt4.attention_prefill(*g, out=out, **kw)
+    graph.replay()
+    torch.cuda.synchronize()
+    own = host(out)
+    del graph
+    assert np.array_equal(np.isnan(staged), np.isnan(own))
+    fine = ~np.isnan(own)
+    assert np.array_equal(staged[fine].view(np.uint32), own[fine].view(np.uint32))
+    assert fine.all() != odd and np.isfinite(own).mean() > 0.5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,n_kv,H,KVH,splits", [
     (64, 1000, 2, 1, (2, 4, 5, 8, 9, 16, 17, 40, 64)),   # combining launch; 16 tiles: empty splits above 16
     (320, 460, 64, 8, (2, 3, 4, 5)),                     # 640+ workgroups: combined by the last split up to 4
