@@ -8,29 +8,6 @@
 
 namespace rt4 {
 
-namespace {
-
-// int4 code of x / s (s = amax/7 or 1), same IEEE ops as the reference quantizers.
-__device__ __forceinline__ uint32_t code4(float x, float s) {
-    return (uint32_t)clampi((int)lrintf(x / s), -8, 7) & 0xFu;
-}
-// The codes of 8 values as one dword (value e in nibble e), x / s taken through
-// the reciprocal when every scale of the wave allows it (bit-equal to code4).
-__device__ __forceinline__ uint32_t codes8(const float* v, float s) {
-    uint32_t w = 0;
-    if (__all(recip_div_ok(s))) {
-        const float y = 1.f / s;
-#pragma unroll
-        for (int e = 0; e < 8; e++) w |= ((uint32_t)clampi((int)lrintf(div_by_recip(v[e], s, y)), -8, 7) & 0xFu) << (4 * e);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++) w |= code4(v[e], s) << (4 * e);
-    }
-    return w;
-}
-
-}  // namespace
-
 // ------------------------------------------------------------------ feeders --
 
 // Q of all heads (restates attn_q_quant_k, src/k_new.hip:228-253): x f32 [T][H][D]

@@ -205,13 +205,7 @@ __global__ __launch_bounds__(512) void quant_rows_a4_k(const float* __restrict__
     for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
     amax = run_max<GL>(amax);
     const float s = amax > 0.f ? amax / 7.f : 1.f;
-    uint32_t w = 0;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const int cc = clampi((int)lrintf(v[e] / s), -8, 7);
-        w |= (uint32_t)(cc & 0xF) << (4 * e);
-    }
-    q[(size_t)r * (K >> 3) + i] = w;
+    q[(size_t)r * (K >> 3) + i] = codes8(v, s);
     if (i % GL == 0) sc[(size_t)(i / GL) * rows + r] = s;
 }
 
@@ -347,10 +341,7 @@ __global__ __launch_bounds__(256) void quant_act_a4_k(const float* __restrict__ 
     for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
     amax = run_max<4>(amax);
     const float s = amax > 0.f ? amax / 7.f : 1.f;
-    uint32_t w = 0;
-#pragma unroll
-    for (int e = 0; e < 8; e++) w |= ((uint32_t)clampi((int)lrintf(v[e] / s), -8, 7) & 0xFu) << (4 * e);
-    aq[(size_t)m * (K >> 3) + i] = w;
+    aq[(size_t)m * (K >> 3) + i] = codes8(v, s);
     if ((i & 3) == 0) sa[(size_t)m * (K >> 5) + (i >> 2)] = s;
 }
 
