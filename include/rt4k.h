@@ -147,9 +147,9 @@ int rt4_gemv_w4a8_groupsums(int32_t* gsum, float* y, const uint32_t* wq, const u
 /* The whole decode linear: quantize x per (row, 128-group) to int8, then the
  * GEMV.  Replaces k_gemv_w4a8 (src/kernels.h:27, src/k_gemv.hip:53-106), which
  * is two launches (quant_act, then the GEMV), as is this one, except that one row
- * of moderate K is one launch that quantizes inside (same codes and scales; the
- * fp32 sums over groups may run in another order than rt4_gemv_w4a8_q's).  x f32
- * [rows][K] contiguous.  The quantized activations go to library-owned
+ * of moderate K, where y is not in x's memory, is one launch that quantizes inside
+ * (same codes and scales; the fp32 sums over groups may run in another order than
+ * rt4_gemv_w4a8_q's).  x f32 [rows][K] contiguous.  The quantized activations go to library-owned
  * scratch, grown with hipMalloc on first use per device (as the reference
  * does, src/k_gemv.hip:56-67); not re-entrant across threads. */
 int rt4_gemv_w4a8(float* y, const uint32_t* wq, const uint16_t* ws, const float* x, int rows,

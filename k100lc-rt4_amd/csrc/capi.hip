@@ -447,6 +447,15 @@ int rt4_gemv_w4a8_cfg(float* y, const uint32_t* wq, const uint16_t* ws, const fl
                     as_stream(stream));
 }
 
+// Waves of the one-launch form for this linear, 0 where it takes two launches: more rows,
+// sizes where the launches are faster, and y in x's memory (an in-place square linear),
+// since a workgroup would store y where another has yet to read x.
+static int row_waves(const float* y, const float* x, int rows, int N, int K, int cus) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(y), b = reinterpret_cast<uintptr_t>(x);
+    if (rows != 1 || (a < b + (size_t)K * sizeof(float) && b < a + (size_t)N * sizeof(float))) return 0;
+    return rt4::gemv_row_waves(N, K, cus);
+}
+
 int rt4_gemv_w4a8(float* y, const uint32_t* wq, const uint16_t* ws, const float* x, int rows,
                   int N, int K, void* stream) {
     if (!y || !wq || !ws || !x) return fail(RT4_E_ARG, "rt4_gemv_w4a8: null pointer");
@@ -465,7 +474,7 @@ int rt4_gemv_w4a8(float* y, const uint32_t* wq, const uint16_t* ws, const float*
     void *q = nullptr, *s = nullptr;
     if ((rc = lib_scratch(kSlotActQ, (size_t)rows * K, &q, st))) return rc;
     if ((rc = lib_scratch(kSlotActS, (size_t)rows * (K / 128) * sizeof(float), &s, st))) return rc;
-    if (const int waves = rows == 1 ? rt4::gemv_row_waves(N, K, cus) : 0)
+    if (const int waves = row_waves(y, x, rows, N, K, cus))
         return hip_status(rt4::launch_gemv_row(y, wq, ws, x, N, K, waves, st), "k_gemv_w4a8 launch");
     hipError_t e = rt4::launch_quant_act_a8(static_cast<int8_t*>(q), static_cast<float*>(s), nullptr, x, rows, K, st);
     if (e != hipSuccess) return hip_status(e, "k_gemv_w4a8 quant launch");
@@ -494,7 +503,7 @@ int rt4_gemv_w4a8_noalloc(float* y, const uint32_t* wq, const uint16_t* ws, cons
     if ((rc = noalloc_scratch(&p, st))) return rc;
     int8_t* q = reinterpret_cast<int8_t*>(p);
     float* s = reinterpret_cast<float*>(p + kNaQ);
-    if (const int waves = rows == 1 ? rt4::gemv_row_waves(N, K, cus) : 0)
+    if (const int waves = row_waves(y, x, rows, N, K, cus))
         return hip_status(rt4::launch_gemv_row(y, wq, ws, x, N, K, waves, st), "rt4_gemv_w4a8_noalloc launch");
     // the same launches and the same split as rt4_gemv_w4a8, so y is bit-identical
     hipError_t e = rt4::launch_quant_act_a8(q, s, nullptr, x, rows, K, st);

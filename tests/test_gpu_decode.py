@@ -158,6 +158,25 @@ def test_gemv_one_row_one_launch(rt4, orc, torch_gpu, N, K, unaligned):
     assert rel_l2(host(y), orc.gemv_w4a8(c["wq"], c["ws"], x_np)) < TIGHT
 
 
+@pytest.mark.parametrize("N,K,off", [(5120, 5120, 0), (300, 5120, 5119), (300, 5120, -299), (9000, 1280, 0)])
+def test_gemv_one_row_in_place(rt4, torch_gpu, N, K, off):
+    """y inside x's memory (off: y's first element past x's, in elements) is the result of separate buffers: every
+    read of x precedes every store of y, in the allocating and in the static-scratch entry."""
+    print(f"case gemv_row in place N={N} K={K} off={off}", flush=True)
+    c = workload.gemv_case(seed=6, M=1, N=N, K=K)
+    wq, ws = dev(torch_gpu, c["wq"]), dev(torch_gpu, c["ws"])
+    x0 = torch_gpu.from_numpy(c["x"]).cuda()
+    want = host(rt4.gemv_w4a8_q(wq, ws, *rt4.quant_act_a8(x0)))
+    buf = torch_gpu.empty(2 * (N + K), dtype=torch_gpu.float32, device="cuda")
+    x, y = buf[N:N + K].view(1, K), buf[N + off:N + off + N].view(1, N)
+    st = torch_gpu.cuda.current_stream().cuda_stream
+    for f in ("rt4_gemv_w4a8", "rt4_gemv_w4a8_noalloc"):
+        x.copy_(x0)
+        assert getattr(rt4.lib(), f)(y.data_ptr(), wq.data_ptr(), ws.data_ptr(), x.data_ptr(), 1, N, K, st) == 0
+        torch_gpu.cuda.synchronize()
+        assert np.array_equal(host(y).view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("M,N,K,gpw,waves", [(4, 300, 3072, 4, 6), (1, 17, 128, 2, 1), (2, 40, 512, 4, 1),
                                              (3, 1000, 5120, 4, 8), (4, 4176, 8192, 4, 8), (1, 520, 2944, 10, 2),
                                              (4, 64, 40960, 8, 16), (2, 48, 1920, 12, 1), (4, 33, 1408, 6, 2)])
