@@ -240,7 +240,7 @@ def gemv_w4a8(wq, ws, x, out=None, groups_per_wave: int = 0, waves: int = 0, k_s
               row_blocks: int = 0):
     """Drop-in k_gemv_w4a8: quantize x f32 [rows, K] and multiply (rows <= 4).
 
-    Two launches (quantizer, GEMV).  A launch configuration (see gemv_w4a8_q)
+    Two launches (quantizer, GEMV), or one for a single row of moderate K.  A launch configuration (see gemv_w4a8_q)
     selects rt4_gemv_w4a8_cfg instead: one launch that quantizes inside the GEMV
     (x 16-byte aligned), bit-identical output."""
     rows, K = x.shape

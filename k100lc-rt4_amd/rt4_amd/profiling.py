@@ -51,7 +51,7 @@ COPY_KERNEL = "copy_k("          # the probe library's plain copy kernel
 KERNELS = {                       # report key -> substring of the rocprof kernel name
     "gemv_gate_up": "gemv_w4a8_tl_k<4",
     "gemv_c0": "gemv_w4a8_dot_k<2, 5",
-    "gemm_gate_up": "gemm_w4a8_k<false>",
+    "gemm_gate_up": "gemm_w4a8_k<",
     "attention_c4": "fa_int4_k",
     "attention_c4_staging": "fa_expand_kv_k",
 }
