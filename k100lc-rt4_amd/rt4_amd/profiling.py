@@ -92,9 +92,9 @@ def attention_bytes(n_q: int, n_kv: int, H: int, KVH: int, D: int = 256) -> dict
 
 def attention_staging_bytes(n_kv: int, KVH: int, D: int = 256) -> int:
     """The prefill's K/V staging pass: the int4 K and V codes read once and their
-    staged operand bytes (16 KB per 64-key tile each for K and V) written once."""
+    staged operand bytes (12 KB per 64-key tile each for K and V) written once."""
     n_tile = (n_kv + 63) // 64
-    return 2 * KVH * n_kv * D // 2 + 2 * KVH * n_tile * 16384
+    return 2 * KVH * n_kv * D // 2 + 2 * KVH * n_tile * 12288
 
 
 ALGO_BYTES = {
