@@ -168,6 +168,10 @@ __device__ __forceinline__ void e2m3_operand(const uint32_t (&w)[4], uint32_t (&
 // max that returns NaN if an operand is one (fmaxf drops it).
 __device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 
+// Output of combined splits, o / l.  A row without a visible key (l = 0) takes o * 0 = 0, and so does a NaN l, whose o is
+// NaN (the P scale carries it into every dim): a non-finite scale leaves the row NaN, as with one split.
+__device__ __forceinline__ float o_over_l(float o, float l) { return l > 0.f ? o / l : o * 0.f; }
+
 // Key order within a 16-key subtile: output register r of lane group G holds key
 // key_of_slot(G, r); the K row fed to the MFMA at slot 4G + r is that key.
 __device__ __forceinline__ int key_of_slot(int G, int r) { return 8 * (G >> 1) + 2 * r + (G & 1); }
@@ -870,8 +874,8 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
 #pragma unroll
             for (int dt = 0; dt < 16; dt++)
                 *reinterpret_cast<float4*>(orow + 16 * dt) =
-                    make_float4(l > 0.f ? o[dt][0] / l : 0.f, l > 0.f ? o[dt][1] / l : 0.f,
-                                l > 0.f ? o[dt][2] / l : 0.f, l > 0.f ? o[dt][3] / l : 0.f);
+                    make_float4(o_over_l(o[dt][0], l), o_over_l(o[dt][1], l), o_over_l(o[dt][2], l),
+                                o_over_l(o[dt][3], l));
             if (tid == 0) __hip_atomic_store(cnt + item, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
@@ -908,8 +912,7 @@ __global__ __launch_bounds__(256) void fa_combine_k(const float* __restrict__ op
                 acc.y = fmaf(as, v[j].y, acc.y);
             }
     }
-    *reinterpret_cast<float2*>(out + (size_t)row * HD + d) =
-        make_float2(l > 0.f ? acc.x / l : 0.f, l > 0.f ? acc.y / l : 0.f);
+    *reinterpret_cast<float2*>(out + (size_t)row * HD + d) = make_float2(o_over_l(acc.x, l), o_over_l(acc.y, l));
 }
 
 // Staged K/V blocks of every tile of every KV head, for the DMA path, made once per call

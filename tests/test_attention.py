@@ -587,6 +587,37 @@ def test_attention_split_combines(rt4, torch_gpu, T, n_kv, H, KVH, splits):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,n_kv,H,KVH,splits", [
+    (64, 1000, 2, 1, (0, 2, 8, 16)),                     # combining launch
+    (320, 460, 64, 8, (2, 3, 4)),                        # combined by the last split
+])
+def test_attention_split_combines_keep_nan(rt4, torch_gpu, T, n_kv, H, KVH, splits):
+    """A row that a NaN or infinite scale makes NaN with one split is NaN however its splits are combined (and no other
+    element is), for a Q scale, a K scale that only one split sees, and a V scale."""
+    torch = torch_gpu
+    print(f"case split combines keep NaN T={T} n_kv={n_kv} H={H} KVH={KVH}", flush=True)
+    rng = np.random.default_rng(43)
+    q, k, v = workload.attn_np(rng, T, n_kv, H, KVH)
+    cap = (n_kv + 63) // 64 * 64
+    g = gpu_cache(rt4, torch, q, k, v, T, cap)
+    qs, ksc, vsc = g[1], g[3], g[5]
+    qs[0, 0, 5], qs[1, 1, 20], qs[1, 0, 33] = float("nan"), float("inf"), 0.0
+    kw = dict(n_kv=n_kv, off=n_kv - T, ratio=H // KVH)
+    for name, scales in (("Q", {}), ("K NaN", {(ksc, (0, 0, n_kv - 3)): float("nan")}),
+                         ("K inf", {(ksc, (KVH - 1, 1, n_kv - T + 30)): float("inf")}),
+                         ("V", {(vsc, (0, 1, 17)): float("nan"), (vsc, (0, 3, 200)): float("inf")})):
+        for (t, at), x in scales.items():
+            t[at] = x
+        one = host(rt4.attention_prefill(*g[:6], kv_splits=1, **kw))
+        assert np.isnan(one[0, 5]).all() and np.isnan(one[1, 20]).all() and np.isfinite(one).mean() > 0.5
+        for s in splits:
+            got = host(rt4.attention_prefill(*g[:6], kv_splits=s, out=torch.full((H, T, HD), 7.0, device="cuda"), **kw))
+            assert np.array_equal(np.isnan(got), np.isnan(one)), f"{name} scales, kv_splits={s}"
+            fine = np.isfinite(one)
+            assert np.array_equal(np.isfinite(got), fine) and rel_l2(got[fine], one[fine]) < 64 * 2.0 ** -23
+
+
+@pytest.mark.gpu
 def test_attention_benchmark_shape_sampled(rt4, orc, torch_gpu):
     """24 heads, GQA 6:1, 1024 queries over a 32768-token cache."""
     c4 = workload.ATTN_C4
