@@ -741,12 +741,17 @@ int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, 
         while (plan.nsplit > 1 && !fits(plan))
             plan = rt4::fa_plan(n_q, n_heads, ratio, off, n_tile, cus, plan.nsplit - 1);
     }
+    // The counters are sized by every eager call with several splits, also one whose own
+    // combine needs none: what may be captured afterwards (fewer splits, which may combine
+    // in the same launch) then depends on its size and not on its form.
     void *part = nullptr, *cnt = nullptr;
+    const size_t cb = rt4::fa_cnt_bytes(n_q, n_heads, plan.nsplit);
     if (plan.nsplit > 1 &&
         ((rc = lib_scratch(kSlotAttnPart, rt4::fa_part_bytes(n_q, n_heads, plan.nsplit), &part, st)) ||
-         (plan.inline_combine &&
-          (rc = lib_scratch(kSlotAttnCnt, rt4::fa_cnt_bytes(n_q, n_heads, plan.nsplit), &cnt, st, true)))))
+         ((plan.inline_combine || !(scratch_has(kSlotAttnCnt, cb) || capturing(st))) &&
+          (rc = lib_scratch(kSlotAttnCnt, cb, &cnt, st, true)))))
         return rc;
+    if (!plan.inline_combine) cnt = nullptr;
     // The staged K/V copy for the DMA form (one staging pass per call instead of per
     // workgroup), where it pays and up to kMaxKvxBytes; beyond that, or under capture while
     // the copy would have to grow, each workgroup stages its own tiles (same results).

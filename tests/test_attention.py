@@ -618,6 +618,33 @@ def test_attention_split_combines_keep_nan(rt4, torch_gpu, T, n_kv, H, KVH, spli
 
 
 @pytest.mark.gpu
+def test_attention_capture_of_fewer_splits_than_an_eager_call(rt4, torch_gpu):
+    """An eager call sizes the workspace of every smaller split count: 5 splits of this grid take the combining launch,
+    2 the combine in the same launch, whose counters must be there when 2 are captured."""
+    torch = torch_gpu
+    T, n_kv, H, KVH = 320, 460, 64, 8
+    print(f"case capture of fewer splits T={T} n_kv={n_kv} H={H}", flush=True)
+    q, k, v = workload.attn_np(np.random.default_rng(47), T, n_kv, H, KVH)
+    g = gpu_cache(rt4, torch, q, k, v, T, 512)
+    kw = dict(n_kv=n_kv, off=n_kv - T, ratio=H // KVH)
+    want = rt4.attention_prefill(*g[:6], kv_splits=2, **kw)
+    torch.cuda.synchronize()
+    rt4.release_scratch()
+    rt4.attention_prefill(*g[:6], kv_splits=5, **kw)
+    torch.cuda.synchronize()
+    out = torch.empty((H, T, HD), dtype=torch.float32, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rt4.attention_prefill(*g[:6], kv_splits=2, out=out, **kw)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.gpu
 def test_attention_benchmark_shape_sampled(rt4, orc, torch_gpu):
     """24 heads, GQA 6:1, 1024 queries over a 32768-token cache."""
     c4 = workload.ATTN_C4
