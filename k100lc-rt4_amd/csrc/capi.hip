@@ -468,14 +468,18 @@ int rt4_gemv_w4a8(float* y, const uint32_t* wq, const uint16_t* ws, const float*
     const rt4::GemvCfg c = rt4::gemv_default_cfg(rows, N, K, cus);
     // Two launches, as the reference: the activation quantizer into library scratch,
     // then the GEMV.  One row, where it is faster: one launch that quantizes in every
-    // workgroup; it needs no scratch, which is sized all the same, so that what may be
-    // captured after a call does not depend on the form.
+    // workgroup; it needs no scratch, which is sized all the same, the split workspace of
+    // the two launches included, so that what may be captured after a call, and how, does
+    // not depend on the form.
     hipStream_t st = as_stream(stream);
     void *q = nullptr, *s = nullptr;
     if ((rc = lib_scratch(kSlotActQ, (size_t)rows * K, &q, st))) return rc;
     if ((rc = lib_scratch(kSlotActS, (size_t)rows * (K / 128) * sizeof(float), &s, st))) return rc;
-    if (const int waves = row_waves(y, x, rows, N, K, cus))
+    if (const int waves = row_waves(y, x, rows, N, K, cus)) {
+        rt4::GemvSplit sp = rt4::gemv_split(N, K, c, cus);
+        if ((rc = gemv_split_ws(&sp, cus, st))) return rc;
         return hip_status(rt4::launch_gemv_row(y, wq, ws, x, N, K, waves, st), "k_gemv_w4a8 launch");
+    }
     hipError_t e = rt4::launch_quant_act_a8(static_cast<int8_t*>(q), static_cast<float*>(s), nullptr, x, rows, K, st);
     if (e != hipSuccess) return hip_status(e, "k_gemv_w4a8 quant launch");
     return run_gemv("k_gemv_w4a8 launch", nullptr, y, wq, ws, static_cast<const int8_t*>(q),

@@ -158,6 +158,32 @@ def test_gemv_one_row_one_launch(rt4, orc, torch_gpu, N, K, unaligned):
     assert rel_l2(host(y), orc.gemv_w4a8(c["wq"], c["ws"], x_np)) < TIGHT
 
 
+def test_gemv_one_row_sizes_the_split_workspace(rt4, torch_gpu):
+    """An eager linear of one row leaves the split workspace that its two launches would use, whichever form it takes:
+    the pre-quantized GEMV captured after it at a shape that is split gives the eager call's bits."""
+    N, K = 300, 12288
+    print(f"case gemv_row split workspace N={N} K={K}", flush=True)
+    c = workload.gemv_case(seed=8, M=1, N=N, K=K)
+    wq, ws, x = dev(torch_gpu, c["wq"]), dev(torch_gpu, c["ws"]), dev(torch_gpu, c["x"])
+    assert rt4.gemv_launch_plan(1, N, K)["k_splits"] > 1
+    xq, sa = rt4.quant_act_a8(x)
+    want = host(rt4.gemv_w4a8_q(wq, ws, xq, sa))
+    torch_gpu.cuda.synchronize()
+    rt4.release_scratch()
+    rt4.gemv_w4a8(wq, ws, x)
+    torch_gpu.cuda.synchronize()
+    y = torch_gpu.empty((1, N), dtype=torch_gpu.float32, device="cuda")
+    graph = torch_gpu.cuda.CUDAGraph()
+    with torch_gpu.cuda.graph(graph):
+        rt4.gemv_w4a8_q(wq, ws, xq, sa, out=y)
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch_gpu.cuda.synchronize()
+        graph.replay()
+        torch_gpu.cuda.synchronize()
+        assert np.array_equal(host(y).view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("N,K,off", [(5120, 5120, 0), (300, 5120, 5119), (300, 5120, -299), (9000, 1280, 0)])
 def test_gemv_one_row_in_place(rt4, torch_gpu, N, K, off):
     """y inside x's memory (off: y's first element past x's, in elements) is the result of separate buffers: every
