@@ -196,13 +196,22 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
     const int lr = lane & 31, lh = lane >> 5;
     const int NG = K >> 7;
     const int P = gridDim.x;
-    const int b = (P % 8 == 0) ? (int)(blockIdx.x % 8) * (P / 8) + (int)(blockIdx.x / 8) : (int)blockIdx.x;
+    // b: this workgroup's number, consecutive ones on one XCD (workgroups are dealt to the
+    // eight XCDs in turn).  rg: its range of the remainder tiles' units, -1 for none: b, or
+    // (sch.spread) the ranges dealt evenly to the XCDs, consecutive ones on one XCD.
+    const int x = (int)(blockIdx.x % 8u), j = (int)(blockIdx.x / 8u);
+    const int b = P % 8 == 0 ? x * (P / 8) + j : (int)blockIdx.x;
+    int rg = b < sch.Pr ? b : -1;
+    if (sch.spread) {
+        const int pq = sch.Pr >> 3, pr = sch.Pr & 7;
+        rg = j < pq + (x < pr ? 1 : 0) ? x * pq + min(x, pr) + j : -1;
+    }
     // This workgroup's work: its range [r0, r1) of the remainder tiles' units (the first
-    // sch.rem tiles, shared by the first sch.Pr workgroups), then sch.full whole tiles,
-    // P apart.  rl_t, rl_e: the last remainder tile of the range and the group it ends
-    // before (-1: no range).
+    // sch.rem tiles, shared by sch.Pr workgroups), then sch.full whole tiles, P apart.
+    // rl_t, rl_e: the last remainder tile of the range and the group it ends before (-1:
+    // no range).
     const int ntm = sch.ntm;
-    const int r0 = b < sch.Pr ? range_start(sch, b) : 0, r1 = b < sch.Pr ? range_start(sch, b + 1) : 0;
+    const int r0 = rg >= 0 ? range_start(sch, rg) : 0, r1 = rg >= 0 ? range_start(sch, rg + 1) : 0;
     const int n = r1 - r0 + sch.full * NG;
     if (n == 0) return;
     const int rl_t = r1 > r0 ? (r1 - 1) / NG : -1, rl_e = r1 > r0 ? r1 - rl_t * NG : 0;
@@ -320,13 +329,13 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
         }
     };
     // End of this workgroup's segment of tile x.t: a whole tile is written out; a part
-    // of one goes to its partial slot, 2b for this workgroup's first tile and 2b + 1 for
+    // of one goes to its partial slot, 2 rg for this workgroup's first tile and 2 rg + 1 for
     // its last remainder tile, for gemm_combine_k.  Nothing is waited for here.
     auto flush = [&](const TileRef& x, bool whole) __attribute__((always_inline)) {
         if (whole) {
             write_c(facc, x.bm, x.bn);
         } else {
-            const __amdgpu_buffer_rsrc_t rs = part_rsrc<RT>(part, 2 * b + (x.t == t_first ? 0 : 1));
+            const __amdgpu_buffer_rsrc_t rs = part_rsrc<RT>(part, 2 * rg + (x.t == t_first ? 0 : 1));
 #pragma unroll
             for (int ii = 0; ii < RT; ii++)
 #pragma unroll
@@ -660,6 +669,14 @@ GemmPlan gemm_plan(int M, int N, int K, int cus) {
         p.s.Pr = p.P;
         p.split = true;
     }
+    // Whether the ranges are spread over the XCDs.  On the first Pr workgroups they load
+    // some XCDs with all of the shared tiles while the others idle or wait; but where they
+    // are less than about three quarters of one XCD's workgroups, one XCD takes them as
+    // fast and reads their operands once.  Measured (us, first workgroups -> spread):
+    // M=1024 N=4096 K=256 (Pr 128) 11.4 -> 9.3, M=946 N=11400 K=128 (104) 14.9 -> 12.8,
+    // M=512 N=18432 K=128 (32) 13.0 -> 12.1, N=17920 (24) 12.0 -> 11.8, N=17664 (20) 11.8 ->
+    // 12.0, N=17408 (16) 11.2 -> 11.9.
+    p.s.spread = p.P % 8 == 0 && p.s.Pr > 3 * p.P / 32;
     p.s.q = p.s.Pr > 0 ? R / p.s.Pr : 0;
     p.s.r = p.s.Pr > 0 ? R % p.s.Pr : 0;
     // two partials of a 128-row tile per workgroup, whatever the tile: one size serves

@@ -89,6 +89,7 @@ struct GemmSched {
     int rem;       // tiles whose K groups are shared out evenly
     int Pr;        // workgroups that share them
     int q, r;      // their (tile, group) units, rem * K/128, over Pr: quotient and remainder
+    int spread;    // whether those workgroups are spread over the XCDs, or the first Pr
 };
 struct GemmPlan {
     int rt;        // 32-row tiles per workgroup tile: 1, 2 or 4

@@ -146,6 +146,17 @@ def test_gemm_row_tiles_and_schedules(rt4, orc, torch_gpu, M, N, K):
     assert rel_l2(y[mi, ni], ref) < TIGHT
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (128, 71680, 128), (128, 71936, 128),    # one whole tile each after 24 (one XCD's) or 25 shared ones (spread)
+    (100, 9472, 1024), (33, 6400, 1408),     # no whole tiles: 37 and 25 tiles in pieces, a piece count not a multiple of 8
+    (640, 65536, 256),                       # 1280 tiles: none shared
+])
+def test_gemm_shared_tiles_over_the_xcds(rt4, orc, torch_gpu, M, N, K):
+    """The shared tiles' ranges on the first workgroups and spread over the XCDs: every range is taken once, also where
+    their number is no multiple of 8.  Same bound as test_gemm_row_tiles_and_schedules."""
+    test_gemm_row_tiles_and_schedules(rt4, orc, torch_gpu, M, N, K)
+
+
 def test_gemm_dropin_small_c2_uses_library_scratch(rt4, orc, torch_gpu):
     """4*N < K: the recombined codes do not fit in c2, library scratch is used."""
     M, N, K = 128, 64, 1024
