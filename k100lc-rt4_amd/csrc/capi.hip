@@ -35,7 +35,7 @@ hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 // the retired buffers of a slot add up to at most twice its final size.  Not
 // safe for concurrent calls from several threads (the reference's scratch has
 // the same property, src/k_gemv.hip:47-51).
-enum Slot { kSlotActQ = 0, kSlotActS = 1, kSlotGemmA = 2, kSlotGemmPart = 3, kSlotAttnPart = 4, kSlotGemvPart = 5, kSlotGemvCnt = 6, kSlotAttnCnt = 7, kSlotAttnKV = 8, kSlots = 9 };
+enum Slot { kSlotActQ = 0, kSlotActS = 1, kSlotGemmA = 2, kSlotGemmPart = 3, kSlotAttnPart = 4, kSlotGemvPart = 5, kSlotGemvCnt = 6, kSlotAttnCnt = 7, kSlotAttnKV = 8, kSlotGemmCnt = 9, kSlots = 10 };
 constexpr int kMaxDev = 64;
 struct Buf {
     void* p = nullptr;
@@ -151,16 +151,22 @@ int device_cus(int* cus) {
     return RT4_OK;
 }
 
-// The GEMM launch with its library-owned split-tile workspace.
+// The GEMM launch with its library-owned split-tile workspace (and counters; under capture
+// without them, the plan's combining launch).
 int run_gemm(const char* who, int32_t* gsum, float* c, const uint32_t* wq, const float* wsc_gm,
              const int8_t* xq, const float* sc, int M, int N, int K, hipStream_t st) {
     int cus = 0, rc = device_cus(&cus);
     if (rc) return rc;
     const rt4::GemmPlan plan = rt4::gemm_plan(M, N, K, cus);
-    void* part = nullptr;
+    void *part = nullptr, *cnt = nullptr;
     if ((rc = lib_scratch(kSlotGemmPart, plan.part_bytes, &part, st))) return rc;
-    return hip_status(
-        rt4::launch_gemm_w4a8(c, gsum, xq, wq, sc, wsc_gm, M, N, K, plan, static_cast<float*>(part), st), who);
+    const size_t cb = (size_t)cus * sizeof(int);
+    if (plan.inline_combine && !(capturing(st) && !scratch_has(kSlotGemmCnt, cb)) &&
+        (rc = lib_scratch(kSlotGemmCnt, cb, &cnt, st, true)))
+        return rc;
+    return hip_status(rt4::launch_gemm_w4a8(c, gsum, xq, wq, sc, wsc_gm, M, N, K, plan, static_cast<float*>(part),
+                                            static_cast<int*>(cnt), st),
+                      who);
 }
 
 // The GEMV launch with its balanced grid: split tiles need a small partial

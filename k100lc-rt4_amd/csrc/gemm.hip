@@ -66,9 +66,10 @@
 // three segments of a workgroup are whole, where equal ranges over all units ("stream-K"
 // throughout) made two of three split: 64 MB of partials written and read back became 32
 // (144 -> 127 us with the combining below; M=2048 262 -> 249).  A part of a tile goes to
-// a workspace slot and gemm_combine_k sums the parts in workgroup order, so results do
-// not depend on timing and no workgroup waits for another.  Workgroups of one XCD take
-// neighbouring tiles (the same weights).
+// a workspace slot, and the parts are summed in range order, by gemm_combine_k or (INL, see
+// gemm_plan) by the workgroup of the tile that counts in last: results do not depend on
+// timing and no workgroup waits for another.  Workgroups of one XCD take neighbouring
+// tiles (the same weights).
 //
 // Row tiles.  RT = 4 (128 rows) from 65 rows up; RT = 2 and 1 for up to 64 and 32 rows,
 // whose units issue less (a unit of RT = 4 takes ~1.36 us here, RT = 2 0.87, RT = 1 0.60:
@@ -108,12 +109,11 @@ struct Tile {
     static constexpr int PART_FLOATS = NT * 16 * RT;      // one partial tile: 16 RT outputs per thread, [k][thread]
 };
 
-// Split-tile partials go through buffer stores and loads with the device-scope cache
-// policy (sc1, that of agent-scope atomics): the stores write through the per-XCD L2
-// and are in memory once the writer's s_waitcnt has retired them, and the loads read
-// the coherent copy.  All 16 of a thread's stores, and all 16 loads of one
-// contributor's partial, are in flight together: one round trip each where four
-// 16-byte groups with a wait of their own took four.
+// Split-tile partials are written by buffer stores with the device-scope cache policy (sc1,
+// that of agent-scope atomics): they write through the per-XCD L2 and are in memory once
+// the writer's s_waitcnt has retired them.  gemm_combine_k, a launch of its own, reads them
+// with plain loads; a workgroup that sums them in the same launch reads them with sc1, the
+// coherent copy, all 4 RT loads of one part in flight together.
 constexpr int kSc1 = 16;               // cache policy: sc1
 constexpr int kRsrcW3 = 0x00020000;    // dword 3 of a buffer resource: 32-bit data format
 template <int RT>
@@ -178,19 +178,20 @@ struct TileRef {
     int t, bm, bn, g;
 };
 
-template <int RT, bool GSUM>
+template <int RT, bool GSUM, bool INL>
 __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ A,
                                                      const uint32_t* __restrict__ W,
                                                      const float* __restrict__ sa,
                                                      const float* __restrict__ sb,
                                                      float* __restrict__ C,
                                                      int32_t* __restrict__ gsum,
-                                                     float* __restrict__ part, int M, int N, int K,
-                                                     GemmSched sch) {
+                                                     float* __restrict__ part, int* __restrict__ cnt,
+                                                     int M, int N, int K, GemmSched sch) {
     using TL = Tile<RT>;
     constexpr int BM = TL::BM, A_ST = TL::A_ST, DMA_PER_UNIT = TL::DMA_PER_UNIT;
     constexpr int LDS_A = TL::LDS_A, LDS_B = TL::LDS_B, LDS_S = TL::LDS_S;
     __shared__ __align__(16) unsigned char lds[TL::LDS_BYTES];
+    __shared__ int s_last;
     const int lane = threadIdx.x & 63;
     const int w = uniform(threadIdx.x >> 6);
     const int lr = lane & 31, lh = lane >> 5;
@@ -330,7 +331,8 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
     };
     // End of this workgroup's segment of tile x.t: a whole tile is written out; a part
     // of one goes to its partial slot, 2 rg for this workgroup's first tile and 2 rg + 1 for
-    // its last remainder tile, for gemm_combine_k.  Nothing is waited for here.
+    // its last remainder tile, for gemm_combine_k or (INL) the tile's last contributor.  No
+    // other workgroup is waited for.
     auto flush = [&](const TileRef& x, bool whole) __attribute__((always_inline)) {
         if (whole) {
             write_c(facc, x.bm, x.bn);
@@ -344,6 +346,39 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
                         v4u{(unsigned)facc[ii][4 * q], (unsigned)facc[ii][4 * q + 1], (unsigned)facc[ii][4 * q + 2],
                             (unsigned)facc[ii][4 * q + 3]},
                         rs, threadIdx.x * 16, (4 * ii + q) * NT * 16, kSc1);
+            if constexpr (INL) {
+                // counted in for this tile once every wave's stores are in memory; the
+                // workgroup that counts last sums the parts, in range order
+                const int wf = owner_of(sch, x.t * NG), wl = owner_of(sch, x.t * NG + NG - 1);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+                if (threadIdx.x == 0)
+                    s_last = __hip_atomic_fetch_add(cnt + x.t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == wl - wf;
+                __syncthreads();
+                if (s_last) {
+                    const int slot_f = 2 * wf + (range_start(sch, wf) == x.t * NG ? 0 : 1);
+#pragma unroll
+                    for (int ii = 0; ii < RT; ii++)
+#pragma unroll
+                        for (int r = 0; r < 16; r++) facc[ii][r] = 0;
+                    for (int v = wf; v <= wl; v++) {
+                        const __amdgpu_buffer_rsrc_t ps = part_rsrc<RT>(part, v == wf ? slot_f : 2 * v);
+                        v4u p[4 * RT];
+#pragma unroll
+                        for (int e = 0; e < 4 * RT; e++)
+                            p[e] = __builtin_amdgcn_raw_buffer_load_b128(ps, threadIdx.x * 16, e * NT * 16, kSc1);
+#pragma unroll
+                        for (int e = 0; e < 4 * RT; e++)
+#pragma unroll
+                            for (int c = 0; c < 4; c++)
+                                facc[e >> 2][4 * (e & 3) + c] = __float_as_int(
+                                    __int_as_float(facc[e >> 2][4 * (e & 3) + c]) + __uint_as_float(p[e][c]));
+                    }
+                    write_c(facc, x.bm, x.bn);
+                    if (threadIdx.x == 0)
+                        __hip_atomic_store(cnt + x.t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
         }
 #pragma unroll
         for (int ii = 0; ii < RT; ii++)
@@ -585,13 +620,16 @@ __global__ __launch_bounds__(NT, 1) void gemm_w4a8_k(const int8_t* __restrict__ 
     }
 }
 
-// The split tiles: C = 1/16 of the sum of a tile's partials in workgroup order.  Block
+// The split tiles: C = 1/16 of the sum of a tile's partials in range order.  Block
 // (t, y) takes the 64 16-byte pieces 64 y.. of remainder tile t, one per thread: register
 // quad y / 8 of the GEMM's wave y % 8, i.e. 8 rows x 32 columns.  Up to four
-// contributors' loads are in flight per thread.
-// Its own launch, and not the last contributor of each tile within the GEMM: that
-// workgroup read up to 13 partials one round trip after another (8.9-19 us at the end of
-// a 20-34 us launch for 16-64 rows, 15.8 us at M=384 K=17408) while the others were done.
+// contributors' loads are in flight per thread.  Bound by the partials' traffic: M=1024
+// N=5120 K=5120, 54 MB read and 21 MB of C written, takes 12.4 us (6.0 TB/s; blocks of 256
+// threads, two or four pieces a thread measure the same).
+// Its own launch where tiles have many parts, and not the last contributor of each tile
+// within the GEMM: that workgroup read up to 13 partials one after another (8.9-19 us at
+// the end of a 20-34 us launch for 16-64 rows, 15.8 us at M=384 K=17408) while the others
+// were done.  gemm_plan says where the last contributor does it.
 template <int RT>
 __global__ __launch_bounds__(64) void gemm_combine_k(const float* __restrict__ part, float* __restrict__ C, int M,
                                                       int N, int NG, GemmSched sch) {
@@ -642,7 +680,8 @@ GemmPlan gemm_plan(int M, int N, int K, int cus) {
     p.P = T < ncu ? (int)T : ncu;
     p.s.full = ntiles / p.P;
     p.s.rem = ntiles - p.s.full * p.P;
-    const int R = p.s.rem * NG;      // their units (rem < P; K = 128 NG < 2^31, so this fits)
+    const int R = p.s.rem * NG;      // their units: rem < P, and one tile only where
+                                     // K / 128 reaches 2^23 (the limits on M K and N K)
     // How many workgroups share the remainder tiles.  Every tile in S pieces on rem * S
     // workgroups (S = 1: whole tiles, nothing to combine), or equal ranges on all of them
     // (better balanced, but most workgroups then touch two tiles and leave two partials).
@@ -669,6 +708,14 @@ GemmPlan gemm_plan(int M, int N, int K, int cus) {
         p.s.Pr = p.P;
         p.split = true;
     }
+    // Equal ranges of more than half a tile's groups: at most three parts a tile, and tiles
+    // that are finished all through the launch, so the last contributor's sum hides behind
+    // the others' work where a combining launch reads every partial (13 us) at the end.
+    // Measured (us, combining launch -> in the launch, graph replayed): M=1024 N=5120
+    // K=17408 136 -> 131, M=609 N=7395 K=7040 64.0 -> 60.7, M=200 N=17408 K=5120 45.7 -> 44.3.
+    // With more parts it loses: M=1024 N=1024 K=5120 (8 parts) 23 -> 28, M=128 N=17408 K=5120
+    // (68 tiles, 4 or 5) 31.0 -> 32.5.
+    p.inline_combine = p.split && p.rt == 4 && p.s.Pr == p.P && 2 * p.s.rem > p.P;
     // Whether the ranges are spread over the XCDs.  On the first Pr workgroups they load
     // some XCDs with all of the shared tiles while the others idle or wait; but where they
     // are less than about three quarters of one XCD's workgroups, one XCD takes them as
@@ -679,29 +726,33 @@ GemmPlan gemm_plan(int M, int N, int K, int cus) {
     p.s.spread = p.P % 8 == 0 && p.s.Pr > 3 * p.P / 32;
     p.s.q = p.s.Pr > 0 ? R / p.s.Pr : 0;
     p.s.r = p.s.Pr > 0 ? R % p.s.Pr : 0;
-    // two partials of a 128-row tile per workgroup, whatever the tile: one size serves
-    // every shape, so a call at a small shape leaves nothing to grow for a larger one
+    // Two partials of a 128-row tile per workgroup, whatever the tile and whether any is
+    // split: what may be captured after an eager call then depends on the workgroup count
+    // alone, which is the CU count from that many (tile, group) units up.
     p.part_bytes = (size_t)p.P * 2 * Tile<4>::PART_FLOATS * sizeof(float);
     return p;
 }
 
 hipError_t launch_gemm_w4a8(float* C, int32_t* gsum, const int8_t* A, const uint32_t* W,
                             const float* sa, const float* sb, int M, int N, int K, const GemmPlan& p,
-                            float* part, hipStream_t st) {
-#define RT4_GEMM(R)                                                                                            \
-    if (gsum)                                                                                                  \
-        hipLaunchKernelGGL((gemm_w4a8_k<R, true>), dim3(p.P), dim3(NT), 0, st, A, W, sa, sb, C, gsum, part, M, N, K, p.s);  \
-    else                                                                                                       \
-        hipLaunchKernelGGL((gemm_w4a8_k<R, false>), dim3(p.P), dim3(NT), 0, st, A, W, sa, sb, C, gsum, part, M, N, K, p.s); \
+                            float* part, int* cnt, hipStream_t st) {
+#define RT4_GEMM_K(R, G, I) \
+    hipLaunchKernelGGL((gemm_w4a8_k<R, G, I>), dim3(p.P), dim3(NT), 0, st, A, W, sa, sb, C, gsum, part, cnt, M, N, K, p.s)
+#define RT4_GEMM(R)                      \
+    if (gsum) RT4_GEMM_K(R, true, false); \
+    else RT4_GEMM_K(R, false, false);     \
     if (p.split) hipLaunchKernelGGL(gemm_combine_k<R>, dim3(p.s.rem, 32 * R), dim3(64), 0, st, part, C, M, N, K / kGroup, p.s);
     if (p.rt == 1) {
         RT4_GEMM(1)
     } else if (p.rt == 2) {
         RT4_GEMM(2)
+    } else if (p.inline_combine && cnt && !gsum) {
+        RT4_GEMM_K(4, false, true);
     } else {
         RT4_GEMM(4)
     }
 #undef RT4_GEMM
+#undef RT4_GEMM_K
     return hipGetLastError();
 }
 

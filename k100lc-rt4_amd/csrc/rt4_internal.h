@@ -82,7 +82,9 @@ hipError_t launch_gemv_w4a4(float* y, const uint32_t* wq, const uint16_t* ws, co
 // group-major scales sa [K/128][M] and sb [K/128][N]; gsum (optional, tests)
 // receives the exact per-group int32 dot products [M][N][K/128].  The launch is
 // persistent (one workgroup per CU).  `part` (part_bytes) is the workspace of the
-// partial sums of tiles that several workgroups share.
+// partial sums of tiles that several workgroups share; `cnt`, for a plan with
+// inline_combine, one counter per workgroup that must be zero before the first launch
+// (every launch leaves them zero again).  Null: the combining launch (same sums).
 struct GemmSched {
     int ntm;       // row tiles
     int full;      // whole tiles per workgroup; they follow the first rem tiles
@@ -95,13 +97,14 @@ struct GemmPlan {
     int rt;        // 32-row tiles per workgroup tile: 1, 2 or 4
     int P;         // workgroups
     GemmSched s;
-    bool split;    // some tile has several contributors: a combining launch follows
+    bool split;    // some tile has several contributors: a combining launch follows,
+    bool inline_combine;   // or the last of them sums the parts in the same launch
     size_t part_bytes;
 };
 GemmPlan gemm_plan(int M, int N, int K, int cus);
 hipError_t launch_gemm_w4a8(float* C, int32_t* gsum, const int8_t* A, const uint32_t* W,
                             const float* sa, const float* sb, int M, int N, int K, const GemmPlan& plan,
-                            float* part, hipStream_t st);
+                            float* part, int* cnt, hipStream_t st);
 hipError_t launch_zero_i32(int* p, size_t n, hipStream_t st);
 
 // ---- int4-KV attention (attn.hip); head dim 256, Q/K groups of 128, V tiles of 64 keys

@@ -157,6 +157,43 @@ def test_gemm_shared_tiles_over_the_xcds(rt4, orc, torch_gpu, M, N, K):
     test_gemm_row_tiles_and_schedules(rt4, orc, torch_gpu, M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1280, 3328, 4096),    # 130 tiles in 256 ranges of 16 or 17 of their 32 groups
+    (609, 7395, 7040),     # 145 tiles, partial rows and columns
+    (640, 19712, 3584),    # 385 tiles: a whole one each after 129 in ranges of 14 or 15 of their 28 groups
+])
+def test_gemm_combines_in_the_launch(rt4, torch_gpu, M, N, K):
+    """Equal ranges of more than half a tile: the last contributor of a tile sums its parts.  The same sums in the same
+    order as the combining launch (which the group-sum entry and a capture without counters take): equal bits."""
+    print(f"case gemm combine in the launch M={M} N={N} K={K}", flush=True)
+    torch = torch_gpu
+    g = torch.Generator(device="cuda").manual_seed(M)
+    wq = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, device="cuda", generator=g).view(torch.int32)
+    sb = torch.rand((K // 128, N), device="cuda", generator=g) * 0.01
+    xq, sc = rt4.quant_rows_i8(torch.randn((M, K), device="cuda", generator=g))
+    outs = [rt4.gemm_w4a8_i8(wq, sb, xq, sc, out=torch.full((M, N), float("nan"), device="cuda")) for _ in range(3)]
+    torch.cuda.synchronize()
+    rt4.release_scratch()
+    x16, s16 = rt4.quant_rows_i8(torch.ones((16, K), device="cuda"))
+    rt4.gemm_w4a8_i8(wq, sb, x16, s16)                 # sizes the partials only
+    torch.cuda.synchronize()
+    out, graph = torch.empty((M, N), device="cuda"), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rt4.gemm_w4a8_i8(wq, sb, xq, sc, out=out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for y in outs:
+            assert torch.equal(y.view(torch.int32), out.view(torch.int32))
+    ref = (xq.view(M, K // 8, 2, 4).transpose(2, 3).reshape(M, K).double() * sc.T.repeat_interleave(128, 1).double())[:64]
+    sh = 4 * torch.arange(8, device="cuda", dtype=torch.int32)
+    w = (((wq[:256].unsqueeze(-1) >> sh) & 15) ^ 8).reshape(256, K).double() - 8
+    ref = ref @ (w * sb[:, :256].T.repeat_interleave(128, 1).double()).T
+    assert ((out[:64, :256] - ref).norm() / ref.norm()).item() < TIGHT
+
+
 def test_gemm_dropin_small_c2_uses_library_scratch(rt4, orc, torch_gpu):
     """4*N < K: the recombined codes do not fit in c2, library scratch is used."""
     M, N, K = 128, 64, 1024
