@@ -1057,6 +1057,9 @@ GemvCfg gemv_mfma_cfg(int rows, int N, int K, int cus) {
     return c;
 }
 
+// Two turns of rows a wave in the one-launch form: many short rows.
+bool row_twice(int N, int K) { return K <= 4096 && N >= 8192; }
+
 // Where the one-launch form (gemv_w4a8_row_k) takes the linear of one fp32 row, and its
 // waves per workgroup: one quantizing turn of the whole row up to K = 8192 (64 lanes x 8
 // elements a wave, rounded up to 4 waves so that they spread evenly over the SIMDs);
@@ -1064,20 +1067,31 @@ GemvCfg gemv_mfma_cfg(int rows, int N, int K, int cus) {
 // a graph (us a call, quantizer launch + GEMV -> this): K=5120 N=5120 6.58 -> 5.66,
 // N=10240 8.7 -> 7.8, N=17408 11.9 -> 10.3 (10 waves: 12.0, 8: 12.4, 16: 12.5), N=40000
 // 20.5 -> 19.9; K=2048 N=1000 4.3 -> 2.8, N=20000 7.7 -> 6.5; K=1024 N=65000 11.4 -> 9.9;
-// K=8192 N=8192 9.9 -> 8.9 (one row a wave; two 9.7), N=28672 22.7 -> 23.0, so not there.
-// Above K = 8192 every workgroup's share of the quantizing grows: K=16384 N=2048 9.95 ->
-// 7.6, K=17408 N=2560 10.1 -> 9.0 but N=5120 12.3 -> 15.6.
+// K=8192 N=4096 1.08x, K=6400 1.20x; K=16384 N=2048 9.4 -> 7.4, K=17408 N=2560 9.6 -> 8.6
+// but N=5120 12.3 -> 15.6 (17408 is the largest K measured).
+// A workgroup of deep rows has its CU to itself and repeats the whole quantizing, so a
+// nearly empty last round of them costs more than the launch it saves:
+//   - K > 6144: one round, up to K = 8192 also two nearly full ones.  K=7168 N=5120 (1.25
+//     rounds) 6.6 us with two launches, 7.6 so, N=8192 (2) 1.01x, N=12288 (3) 0.98x; K=8192
+//     N=8192 1.07x, N=6553 (1.6) 1.01x; K=9216 N=2150 (1.05) 0.87x.
+//   - K > 3072 with 24 rows and more a workgroup: not where less than 0.4 of the second or
+//     third round is filled.  K=5120 N=6758 (1.1) 0.91x, N=7680 (1.25) 0.92x, N=8601 (1.4)
+//     1.00x, N=13516 (2.2) 0.97x, N=20275 (3.3) 1.01x; K=4096 N=9011 (1.1) 0.95x.
 int gemv_row_waves(int N, int K, int cus) {
     const long long ncu = cus > 0 ? cus : 256;
-    if (K % 256) return 0;
-    if (K <= 8192) return (N + 15) / 16 <= 16 * ncu && (K <= 6144 || N <= 64 * ncu) ? 4 * ((K + 2047) / 2048) : 0;
-    if (K > 17408 || N > 10 * ncu) return 0;
-    return K <= 16384 ? 8 : 12;
+    if (K % 256 || K > 17408 || (N + 15) / 16 > 16 * ncu) return 0;
+    if (K > 16384) return N <= 10 * ncu ? 12 : 0;
+    const int waves = K <= 8192 ? 4 * ((K + 2047) / 2048) : 8;
+    const int rows = waves * (K <= 6144 ? 2 : 1) * (row_twice(N, K) ? 2 : 1);
+    const long long wgs = (N + rows - 1) / rows, full = wgs / ncu, last = wgs % ncu;
+    if (K > 6144) return wgs <= ncu || (K <= 8192 && 4 * wgs > 7 * ncu && wgs <= 2 * ncu) ? waves : 0;
+    if (K > 3072 && rows >= 24 && (full == 1 || full == 2) && last > 0 && 5 * last < 2 * ncu) return 0;
+    return waves;
 }
 
 hipError_t launch_gemv_row(float* y, const uint32_t* wq, const uint16_t* ws, const float* xf, int N, int K, int waves,
                            hipStream_t st) {
-    const bool twice = K <= 4096 && N >= 8192;
+    const bool twice = row_twice(N, K);
 #define RT4_ROW(R, NI, IT, XI) return launch_row<R, NI, IT, XI>(y, wq, ws, xf, N, K, waves, st)
     switch ((K + 1023) / 1024) {              // load instructions of two rows
         case 1: if (twice) RT4_ROW(2, 1, 2, 1); RT4_ROW(2, 1, 1, 1);

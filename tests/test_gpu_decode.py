@@ -158,6 +158,14 @@ def test_gemv_one_row_one_launch(rt4, orc, torch_gpu, N, K, unaligned):
     assert rel_l2(host(y), orc.gemv_w4a8(c["wq"], c["ws"], x_np)) < TIGHT
 
 
+@pytest.mark.parametrize("N,K", [(4096, 6400), (4097, 6400), (4096, 8192), (7169, 7168), (2048, 9216), (2049, 9216),     # one round
+                                 (6144, 5120), (6145, 5120), (8592, 4352), (8616, 4352),   # 0.4 of the second round
+                                 (16301, 4096), (8192, 3328), (11468, 3328)])
+def test_gemv_one_row_rounds(rt4, orc, torch_gpu, N, K):
+    """Both sides of the one-launch rule's limits on the workgroups' last round: the same result in either form."""
+    test_gemv_one_row_one_launch(rt4, orc, torch_gpu, N, K, False)
+
+
 def test_gemv_one_row_sizes_the_split_workspace(rt4, torch_gpu):
     """An eager linear of one row leaves the split workspace that its two launches would use, whichever form it takes:
     the pre-quantized GEMV captured after it at a shape that is split gives the eager call's bits."""
