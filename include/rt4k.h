@@ -284,6 +284,14 @@ int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, 
                               int off, int n_tile, int n_heads, int ratio, int kv_cap, int kv_splits,
                               void* stream);
 
+/* How rt4_attention_prefill_cfg runs these sizes on a device of `cus` CUs (0: the
+ * current device, the only case that touches one): the KV splits, whether they are
+ * combined in the same launch (1 for one split), and whether K/V are staged once for
+ * all workgroups; a call under capture without the workspace may take less.  No
+ * counterpart in the reference; for tests and reports. */
+int rt4_attention_launch_plan(int n_q, int n_heads, int ratio, int off, int n_tile, int kv_splits, int cus,
+                              int* splits, int* one_launch, int* staged);
+
 /* ----------------------------------------- W4A4 siblings (RT_ACT4 path) ---- */
 
 /* int4 activation quantizer.  Replaces k_quant_rows (src/kernels.h:36,

@@ -69,9 +69,9 @@
 // block and split, about a tenth of the kernel at C4.  With few tiles a workgroup, or
 // without room for the copy (graph capture before the first eager call, or a copy beyond
 // 4 GiB), each workgroup stages its tiles itself from the packed cache (FP8), with the
-// same products.  The KV range is split over workgroups until the grid fills the CUs (fa_plan),
-// down to three tiles a workgroup; a workgroup starts with one memory round trip (Q and
-// the first tiles' loads together) and converts Q by table look-up (v_perm_b32) while
+// same products.  The KV range is split over workgroups (fa_plan: at most 64 splits, down to
+// one tile each where the grid is small); a workgroup starts with one memory round trip (Q
+// and the first tiles' loads together) and converts Q by table look-up (v_perm_b32) while
 // the tiles arrive (both: C4 645 -> 639 us, 43 rows over 4096 keys 26.2 -> 25.2).
 // Tiles past the workgroup's last query
 // position are skipped: the reference processes them but every entry is masked,
@@ -884,8 +884,9 @@ __global__ __launch_bounds__(NTA, 2) void fa_int4_k(const uint32_t* __restrict__
 // Sum of the KV splits' partial states (fa_plan says when: more than kFaInlineSplits of
 // them, or a grid of one round, where the last split would do it alone at the end, a
 // workgroup reading every partial of 64 rows: of a 44 us call at 64 rows, 24 heads and
-// 4096 keys in 8 splits that was ~13): one wave per half row, two dims a lane.  M = max_s m_s, a_s = 2^(m_s - M), out = Σ_s a_s O_s / Σ_s a_s L_s, the
-// sums in split order.  PB splits' loads are in flight at a time.
+// 4096 keys in 8 splits that was ~13): one wave per half row, two dims a lane.
+// M = max_s m_s, a_s = 2^(m_s - M), out = Σ_s a_s O_s / Σ_s a_s L_s, the O in split order, the
+// L pairwise (every order is fixed).  PB splits' loads are in flight at a time.
 template <int PB>
 __global__ __launch_bounds__(256) void fa_combine_k(const float* __restrict__ opart, const float2* __restrict__ mlpart,
                                                     float* __restrict__ out, int rows, int nsplit) {
@@ -948,47 +949,55 @@ __global__ __launch_bounds__(256) void fa_expand_kv_k(const uint32_t* __restrict
 // -------------------------------------------------------------- launchers --
 
 FaPlan fa_plan(int n_q, int n_heads, int ratio, int off, int n_tile, int cus, int kv_splits) {
-    // The cheapest split count by a cost model (us) fitted to the sweep below: a tile takes
-    // 1.3 us in a workgroup that has its CU to itself and 1.6 where two share one (LDS
-    // allows two), in as many rounds as the grid needs; ~6 us to start and end; the
-    // combining launch 3.5 us and the partials (64 KB a workgroup, written and read) 0.025
-    // each, of which most hides when the last splits combine while others still run.
-    // Measured (one layer, 24 heads over 4 KV heads unless noted; us for the start's rule
-    // of at most 8 splits of at least 8 tiles, balancing rounds only -> this one): 43
-    // rows over 4096 keys 44 -> 25 (10 splits), 100 rows 49 -> 33, 64 rows over 1024 keys
-    // 28.5 -> 17 (6), 6 rows over 25088 keys with 6 heads over one KV head 92 -> 28 (42),
-    // 9 rows over 9472 with 8 over 8 60 -> 23 (32); C4 keeps its 4.
+    // The cheapest split count, staging and combine by a cost model (us) fitted to 490 shapes
+    // (64-1024 rows, 1-528 tiles, 1-64 heads, every count and form timed; it picks within
+    // 0.6% of the best measured on average).  A tile takes `solo` in a workgroup that has
+    // its CU to itself and `pair` where two share one (LDS allows two): less in the staged
+    // form, which costs a launch, ~3.4 us and 5.6 ns a tile and KV head, beforehand.  The
+    // longest workgroup's tiles go in rounds of two workgroups a CU, the last round solo if
+    // it fits; where workgroups differ in length (causal first prompts) the shorter ones
+    // fill in, and the time is the total over the slots plus the shortest; a workgroup of one
+    // tile saves 0.4.  Combining: a launch, and 64 KB of partials a workgroup written and
+    // read; in the same launch those mostly hide.  Measured (us, one layer; a rule that only
+    // balances rounds, at most 8 splits of at least 8 tiles -> this one): 24 heads over 4, 43
+    // rows over 4096 keys 44 -> 25 (10 splits), 64 over 1024 28.5 -> 17 (6); 6 heads over 1,
+    // 6 rows over 25088 keys 92 -> 28 (40); 16 over 4, 896 over 1664 44.0 -> 38.8 (1, staged);
+    // 64 over 8, 640 over 960 54.4 -> 41.5 (1, staged); C4 keeps 4.
+    constexpr double solo[2] = {1.37, 1.04}, pair[2] = {1.76, 1.35};   // FP8 in the workgroups, staged FP6
     cus = cus > 0 ? cus : 256;
     const int items = n_q / QROWS * n_heads, slots = 2 * cus;
-    const int last = (off + n_q - 1) / BNK + 1, nt = last < n_tile ? last : n_tile;   // tiles of the last block
+    const long long last = ((long long)off + n_q - 1) / BNK + 1, first = ((long long)off + QROWS - 1) / BNK + 1;
+    const int nt = last < n_tile ? (int)last : n_tile;       // tiles of the last query block
+    const int nf = first < nt ? (int)first : nt;             // and of the first
+    const double total = 0.5 * ((double)nt + nf) * items, stage = 3.4 + 0.0056 * (double)n_tile * (n_heads / ratio);
     FaPlan p{1, false, false};
-    double best = 0.0;
-    for (int s = 1; s <= kFaMaxSplits && s <= nt; s++) {
-        if (kv_splits > 0 && s != kv_splits && !(s == 1)) continue;
-        const long long blocks = (long long)items * s;
-        const double rounds = (double)((blocks + slots - 1) / slots);
-        const bool in = s > 1 && s <= kFaInlineSplits && blocks > slots;
-        double c = (double)((nt + s - 1) / s) * rounds * (blocks <= cus ? 1.3 : 1.6);
-        if (s > 1) c += 3.5 + (double)blocks * (in ? 0.006 : 0.025);
-        if (s == 1 || s == kv_splits || (kv_splits == 0 && c < best)) {
-            best = c;
-            p.nsplit = s;
-            p.inline_combine = in;
+    double best = -1.0;
+    auto consider = [&](int s) {
+        const double blocks = (double)items * s, full = (double)(long long)(blocks / slots), rem = blocks - full * slots;
+        const double chain = (nt + s - 1) / s, least = (nf + s - 1) / s;
+        const bool in = s > 1 && s <= kFaInlineSplits && blocks >= (s < 4 ? slots : 2 * slots);
+        const double comb = s == 1 ? 0.0 : in ? 7.6 + 0.0164 * blocks : 2.4 + 0.023 * blocks + 0.046 * s;
+        for (int x = 0; x < 2; x++) {
+            double c = chain * (full * pair[x] + (rem == 0 ? 0.0 : rem <= cus ? solo[x] : pair[x]));
+            if (full > 0) {
+                double f = total / slots * pair[x] + least * solo[x];
+                if (f < chain * pair[x]) f = chain * pair[x];
+                if (f < c) c = f;
+            }
+            c += comb + (x ? stage : 0.0) - (chain == 1 ? 0.4 : 0.0);
+            if (best < 0 || c < best) {
+                best = c;
+                p = FaPlan{s, in, x == 1};
+            }
         }
+    };
+    if (kv_splits > 0) {
+        consider(kv_splits);                                 // (more splits than tiles: some are empty)
+        return p;
     }
-    if (kv_splits > 0 && p.nsplit != kv_splits) {       // more splits than tiles: some are empty
-        p.nsplit = kv_splits;
-        p.inline_combine = kv_splits <= kFaInlineSplits && (long long)items * kv_splits > slots;
-    }
-    // Stage K/V once for all (a launch, ~4 us and 5.5 ns a tile and KV head), or in every
-    // workgroup, which costs it 0.3 us a tile (0.45 where two share a CU), the FP8 form's
-    // slower products included.  Measured (us, 24 heads over 4 unless noted, staged / not): 43
-    // rows over 4096 keys 26.6 / 22.4, 128 over 16384 62.3 / 65.4, 256 over 2048 35.6 / 36.0,
-    // 1000 rows alone 32.3 / 33.6, 512 alone 19.8 / 19.4, 64 over 32768 with 8 heads over 8
-    // 60.9 / 36.3, C4 618 / 756.
-    const long long blocks = (long long)items * p.nsplit;
-    const double visits = (double)((nt + p.nsplit - 1) / p.nsplit) * (double)((blocks + slots - 1) / slots);
-    p.staged = visits * (blocks <= cus ? 0.3 : 0.45) > 4.0 + 0.0055 * (double)n_tile * (n_heads / ratio);
+    consider(1);
+    for (int s = 2; s <= kFaMaxSplits && s <= nt && (s <= kFaInlineSplits || (long long)items * s <= 6LL * slots); s++)
+        consider(s);
     return p;
 }
 

@@ -721,6 +721,28 @@ constexpr int kMaxKvCap = (1 << 24) - 64;
 // Largest staged K/V copy the prefill allocates (4 GiB: 174762 tiles x KV heads).
 constexpr size_t kMaxKvxBytes = (size_t)4 << 30;
 
+static rt4::FaPlan attention_plan(int n_q, int n_heads, int ratio, int off, int n_tile, int cus, int kv_splits) {
+    rt4::FaPlan p = rt4::fa_plan(n_q, n_heads, ratio, off, n_tile, cus, kv_splits);
+    p.staged = p.staged && rt4::fa_kvx_bytes(n_heads, ratio, n_tile) <= kMaxKvxBytes;
+    return p;
+}
+
+int rt4_attention_launch_plan(int n_q, int n_heads, int ratio, int off, int n_tile, int kv_splits, int cus,
+                              int* splits, int* one_launch, int* staged) {
+    if (!splits || !one_launch || !staged) return fail(RT4_E_ARG, "rt4_attention_launch_plan: null pointer");
+    if (n_q < 64 || n_q % 64 || off < 0 || n_tile < 1 || n_heads < 1 || ratio < 1 || n_heads % ratio ||
+        n_q > 65535 * 64 || n_heads > 65535 || n_tile > kMaxKvCap / 64 || kv_splits < 0 || kv_splits > 64 || cus < 0)
+        return fail(RT4_E_SHAPE, "rt4_attention_launch_plan: n_q=%d n_heads=%d ratio=%d off=%d n_tile=%d kv_splits=%d cus=%d",
+                    n_q, n_heads, ratio, off, n_tile, kv_splits, cus);
+    int rc;
+    if (cus == 0 && (rc = device_cus(&cus))) return rc;
+    const rt4::FaPlan p = attention_plan(n_q, n_heads, ratio, off, n_tile, cus, kv_splits);
+    *splits = p.nsplit;
+    *one_launch = p.nsplit == 1 || p.inline_combine;
+    *staged = p.staged;
+    return RT4_OK;
+}
+
 int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, const uint32_t* kc,
                               const float* ksc, const uint32_t* vc, const float* vsc, int n_q, int n_kv, int off,
                               int n_tile, int n_heads, int ratio, int kv_cap, int kv_splits, void* stream) {
@@ -739,7 +761,7 @@ int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, 
     int cus = 0, rc = device_cus(&cus);
     if (rc) return rc;
     hipStream_t st = as_stream(stream);
-    rt4::FaPlan plan = rt4::fa_plan(n_q, n_heads, ratio, off, n_tile, cus, kv_splits);
+    rt4::FaPlan plan = attention_plan(n_q, n_heads, ratio, off, n_tile, cus, kv_splits);
     // Under graph capture an automatic split count that would need a larger
     // workspace falls back to the largest count whose workspace is there, down to one
     // split, which needs none (same algorithm, the fp32 sums of O and L in another order).
@@ -749,7 +771,7 @@ int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, 
                    (!p.inline_combine || scratch_has(kSlotAttnCnt, rt4::fa_cnt_bytes(n_q, n_heads, p.nsplit)));
         };
         while (plan.nsplit > 1 && !fits(plan))
-            plan = rt4::fa_plan(n_q, n_heads, ratio, off, n_tile, cus, plan.nsplit - 1);
+            plan = attention_plan(n_q, n_heads, ratio, off, n_tile, cus, plan.nsplit - 1);
     }
     // The counters are sized by every eager call with several splits, also one whose own
     // combine needs none: what may be captured afterwards (fewer splits, which may combine
@@ -763,11 +785,11 @@ int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, 
         return rc;
     if (!plan.inline_combine) cnt = nullptr;
     // The staged K/V copy for the DMA form (one staging pass per call instead of per
-    // workgroup), where it pays and up to kMaxKvxBytes; beyond that, or under capture while
-    // the copy would have to grow, each workgroup stages its own tiles (same results).
+    // workgroup), where the plan has it; under capture while the copy would have to grow,
+    // each workgroup stages its own tiles (same results).
     const size_t xb = rt4::fa_kvx_bytes(n_heads, ratio, n_tile);
     void* kvx = nullptr;
-    if (plan.staged && xb <= kMaxKvxBytes && !(capturing(st) && !scratch_has(kSlotAttnKV, xb)) &&
+    if (plan.staged && !(capturing(st) && !scratch_has(kSlotAttnKV, xb)) &&
         (rc = lib_scratch(kSlotAttnKV, xb, &kvx, st)))
         return rc;
     return hip_status(rt4::launch_fa_int4(out, qq, qsc, kc, ksc, vc, vsc, n_q, n_kv, off, n_tile, n_heads, ratio,

@@ -35,7 +35,7 @@ C_EXPORTS = (
     "rt4_gemm_w4a4",
     "rt4_gemm_w4a8", "rt4_gemm_w4a8_i8", "rt4_gemm_w4a8_groupsums",
     "rt4_attn_q_quant", "rt4_kv_append_k", "rt4_kv_append_v", "rt4_attention_prefill",
-    "rt4_attention_prefill_cfg",
+    "rt4_attention_prefill_cfg", "rt4_attention_launch_plan",
     "rt4_file_open", "rt4_file_close", "rt4_file_count", "rt4_file_find", "rt4_file_info", "rt4_file_data",
     "rt4_file_size", "rt4_file_upload", "rt4_file_upload_tensor",
 )
@@ -89,6 +89,7 @@ _SIGS = {
     "rt4_kv_append_v": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "rt4_attention_prefill": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "rt4_attention_prefill_cfg": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
+    "rt4_attention_launch_plan": [_I, _I, _I, _I, _I, _I, _I, _P, _P, _P],
 }
 
 
@@ -424,6 +425,15 @@ def kv_append_v(vc, vsc, stage, vf, t0: int):
     BG = stage.shape[1]
     _check(lib().rt4_kv_append_v(_ptr(vc), _ptr(vsc), _ptr(stage), _ptr(vf), t0, T, H, D, BG,
                                  vc.shape[1] * 8, _stream()))
+
+
+def attention_launch_plan(n_q: int, n_heads: int, ratio: int, off: int, n_kv: int, kv_splits: int = 0,
+                          cus: int = 0) -> dict:
+    """How attention_prefill runs these sizes on a device of `cus` CUs (0: the current device)."""
+    s, o, g = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    _check(lib().rt4_attention_launch_plan(n_q, n_heads, ratio, off, (n_kv + 63) // 64, kv_splits, cus,
+                                           ctypes.byref(s), ctypes.byref(o), ctypes.byref(g)))
+    return {"splits": s.value, "one_launch": bool(o.value), "staged": bool(g.value)}
 
 
 def attention_prefill(qq, qsc, kc, ksc, vc, vsc, n_kv: int, off: int, ratio: int,

@@ -563,6 +563,38 @@ def test_attention_staged_operands_of_every_code(rt4, torch_gpu, odd):
     assert fine.all() != odd and np.isfinite(own).mean() > 0.5
 
 
+@pytest.mark.parametrize("T,ctx,H,KVH,want", [
+    (1024, 32768, 24, 4, (4, True, True)), (64, 4096, 24, 4, (10, False, False)), (64, 0, 24, 4, (1, True, False)),
+    # sizes where a count that only fills the slots measured slower (us: 53 -> 39, 56 -> 42, 80 -> 42, 61 -> 50)
+    (896, 768, 16, 4, (1, True, True)), (448, 1344, 32, 4, (1, True, True)), (640, 320, 64, 8, (1, True, True)),
+    (448, 1792, 32, 4, (1, True, True)),
+])
+def test_attention_plan_of_measured_sizes(rt4, T, ctx, H, KVH, want):
+    """The plan on 256 CUs is the measured best (or within 2% of it); no GPU is needed to ask."""
+    p = rt4.attention_launch_plan(T, H, H // KVH, ctx, ctx + T, cus=256)
+    assert (p["splits"], p["one_launch"], p["staged"]) == want
+
+
+def test_attention_plan_limits(rt4):
+    """An explicit split count is kept, an automatic one is at most 64 and at most the tiles; only up to 4 splits of
+    a grid beyond two workgroups a CU combine in their launch; a staged copy never exceeds 4 GiB."""
+    rng = np.random.default_rng(3)
+    for _ in range(3000):
+        T, tiles, KVH = 64 * int(rng.integers(1, 40)), int(2 ** rng.uniform(0, 18)), int(rng.integers(1, 9))
+        H, n_kv, s, cus = KVH * int(rng.integers(1, 9)), 64 * tiles, int(rng.choice([0, 0, 1, 2, 3, 4, 5, 17, 64])), 256
+        off = max(0, n_kv - T) if rng.random() < 0.9 else int(rng.integers(0, 2 ** 31))
+        p = rt4.attention_launch_plan(T, H, H // KVH, off, n_kv, s, cus)
+        assert p["splits"] == s if s else 1 <= p["splits"] <= min(64, tiles)
+        if p["splits"] > 1 and p["one_launch"]:
+            assert p["splits"] <= 4 and T // 64 * H * p["splits"] >= 2 * cus
+        if p["staged"]:
+            assert 2 * KVH * tiles * 12288 <= 4 << 30
+    with pytest.raises(rt4.RT4Error):
+        rt4.attention_launch_plan(64, 4, 1, 0, 64, 65, 256)
+    with pytest.raises(rt4.RT4Error):
+        rt4.attention_launch_plan(32, 4, 1, 0, 64, 0, 256)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,n_kv,H,KVH,splits", [
     (64, 1000, 2, 1, (2, 4, 5, 8, 9, 16, 17, 40, 64)),   # combining launch; 16 tiles: empty splits above 16
