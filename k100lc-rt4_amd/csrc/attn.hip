@@ -189,8 +189,6 @@ __device__ __forceinline__ v16f outer16(float x_of_lane, float y) {
     return __builtin_amdgcn_mfma_f32_16x16x1f32(x_of_lane, y, z, 0, 0, 0);
 }
 
-__device__ __forceinline__ int sext4(uint32_t w, int e) { return ((int)(w << (28 - 4 * e))) >> 28; }
-
 constexpr int kRsrcW3 = 0x00020000;    // dword 3 of a buffer resource: 32-bit data format
 
 // The staged form of a 64-key tile: the MFMA operand bytes in the order the waves
