@@ -66,6 +66,7 @@ ONLY = {
     "attn_ref_131k": "FlashAttention prefill, 1024 queries over 131072 cached tokens",
     "gemv_gate_up_m4": "GEMV on quantized activations, M=4 N=17408 K=5120, 16 weight sets",
     "gemv_c0_m1": "GEMV on quantized activations, M=1 N=5120 K=5120, 16 weight sets",
+    "linear_gate_up_m1": "decode linear of one fp32 row, M=1 N=17408 K=5120, 16 weight sets",
 }
 
 
@@ -468,11 +469,16 @@ def only_one(torch, rt4_amd, workload, gen, key: str, launches: int) -> int:
         c = AttnCase(torch, rt4_amd, workload, gen, workload.ATTN_C4 if key == "attn_c4" else workload.ATTN_REF)
         one = lambda i: c.fa(rt4_amd)  # noqa: E731
     else:
-        M, N, K = (4, 17408, 5120) if key == "gemv_gate_up_m4" else (1, 5120, 5120)
+        M, N, K = {"gemv_gate_up_m4": (4, 17408, 5120), "gemv_c0_m1": (1, 5120, 5120),
+                   "linear_gate_up_m1": (1, 17408, 5120)}[key]
         mats = [workload.weights_torch(N, K, generator=gen) for _ in range(16)]
-        xq, sa = rt4_amd.quant_act_a8(workload.acts_torch(M, K, generator=gen))
+        x = workload.acts_torch(M, K, generator=gen)
+        xq, sa = rt4_amd.quant_act_a8(x)
         y = torch.empty((M, N), device="cuda")
-        one = lambda i: rt4_amd.gemv_w4a8_q(*mats[i % 16], xq, sa, out=y)  # noqa: E731
+        if key.startswith("linear_"):
+            one = lambda i: rt4_amd.gemv_w4a8(*mats[i % 16], x, out=y)  # noqa: E731
+        else:
+            one = lambda i: rt4_amd.gemv_w4a8_q(*mats[i % 16], xq, sa, out=y)  # noqa: E731
     one(0)                                   # eager first call: kernel attributes, workspaces
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
@@ -673,7 +679,7 @@ def main() -> int:
             kernels["gemv_c0_m1"]["load_pattern"] = pattern_entry(pat_c0, c0_bytes, c0_us)
         kernels["ceilings"] = {"mfma_i32_16x16x64_i8_TOPS": probe.mfma_i8_rate(torch),
                                "mfma_i32_32x32x32_i8_TOPS": probe.mfma_i8_rate(torch, big=True),
-                               "mfma_f32_16x16x128_fp8_TOPS": probe.mfma_f8_16x16_rate(torch),
+                               **probe.mfma_f8f6_16x16_rates(torch),
                                **probe.mfma_f8f6f4_rates(torch),
                                "gemm_unit_skeleton": probe.gemm_unit_cycles(torch),
                                "graph_node_us": probe.launch_cost(torch, timed_graph),
@@ -688,12 +694,13 @@ def main() -> int:
         kernels.update(gemm_table(torch, rt4_amd, workload, gen))
         kernels.update(attn_table(torch, rt4_amd, workload, gen))
         # the same figures against the MFMA rate measured on this box for the instruction
-        # each kernel runs (the GEMM int8 32x32x32, the attention FP8 16x16x128)
+        # each kernel runs (the GEMM int8 32x32x32, the attention FP6 16x16x128: both shapes
+        # stage K/V)
         for key, rate in (("gemm_c2_gate_up", "mfma_i32_32x32x32_i8_TOPS"),
                           ("gemm_c2_down", "mfma_i32_32x32x32_i8_TOPS"),
                           ("gemm_ref_m2048", "mfma_i32_32x32x32_i8_TOPS"),
-                          ("attn_c4_prefill", "mfma_f32_16x16x128_fp8_TOPS"),
-                          ("attn_ref_131k_prefill", "mfma_f32_16x16x128_fp8_TOPS")):
+                          ("attn_c4_prefill", "mfma_f32_16x16x128_fp6_TOPS"),
+                          ("attn_ref_131k_prefill", "mfma_f32_16x16x128_fp6_TOPS")):
             tops = kernels[key].get("TOPS", kernels[key].get("TOPS_effective"))
             kernels[key]["frac_measured_issue"] = round(tops / kernels["ceilings"][rate], 4)
         lm = [workload.weights_torch(248320, 5120, generator=gen) for _ in range(2)]

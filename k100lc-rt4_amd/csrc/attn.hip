@@ -23,11 +23,12 @@
 // integer codes exactly, so the products come out as fp32 with no int-to-float
 // conversion.  There are two operand forms with the same exact products.  Tiles staged
 // once per call (below) hold FP6 E2M3 operands, code c as c/8: that instruction takes
-// 12.2 cycles where the FP8 one takes 20.2, a tile's operands are 12 KB each of K and V
-// in place of 16, and one v_cvt_scalef32_2xpk16_fp6_f32 packs a lane's 16 P codes in
-// place of eight conversions (C4 661 -> 618 us, 2048 rows over 4096 keys 163 -> 154, 1000
-// rows alone 33.5 -> 32.3).  Packing FP6 takes more instructions than FP8 does, once per
-// call but not once per workgroup, so tiles that a workgroup unpacks itself are FP8 E4M3:
+// 18.3-20 cycles where the FP8 one takes 33-37 (two waves per SIMD, 8 chains each, 2.4
+// GHz), a tile's operands are 12 KB each of K and V in place of 16, and one
+// v_cvt_scalef32_2xpk16_fp6_f32 packs a lane's 16 P codes in place of eight conversions
+// (C4 661 -> 618 us, 2048 rows over 4096 keys 163 -> 154, 1000 rows alone 33.5 -> 32.3).
+// Packing FP6 takes more instructions than FP8 does, once per call but not once per
+// workgroup, so tiles that a workgroup unpacks itself are FP8 E4M3:
 //   - K and V codes c enter as the byte c + 8 (the nibble xor 8), which is the
 //     E4M3 encoding of (c + 8)·2^-9: the subnormals 0..7 and the first normal
 //     binade 8..15 are spaced 2^-9 apart.  The offset's contribution, 8 times the

@@ -27,7 +27,8 @@
 //   rt4p_mfma_f8f6f4 back-to-back v_mfma_scale_f32_32x32x64_f8f6f4 with FP8, FP6 or
 //                   FP4 operands (the matrix-core rate per format)
 //   rt4p_mfma_f8_16x16 back-to-back v_mfma_f32_16x16x128_f8f6f4 (FP8, no block
-//                   scale), the form the attention kernel issues, 8 chains per wave
+//                   scale), the form the attention's unstaged tiles take, 8 chains per wave
+//   rt4p_mfma_f6_16x16 the same with FP6 E2M3 operands, the form its staged tiles take
 //   rt4p_gemm_unit  the prefill GEMM's per-unit instruction skeleton without memory:
 //                   per wave and 128-wide K group, four 32x32 row tiles of MFMAs with
 //                   the previous row tile's fold interleaved, at the GEMM's occupancy
@@ -343,9 +344,10 @@ hipError_t launch_gemv_loads(const uint32_t* wq, const uint16_t* ws, const int8_
 __global__ void empty_k() {}
 
 // ---- scaled f8f6f4 MFMA rate: four independent accumulator chains per wave.
-// 8 independent chains of the unscaled 16x16x128 FP8 MFMA per wave (the scale
-// builtin with zero scales compiles to the unscaled instruction).
-__global__ __launch_bounds__(512) void mfma_f8_16_k(float* __restrict__ sink, int iters, int seed) {
+// 8 independent chains of the unscaled 16x16x128 FP8 (FMT 0) or FP6 E2M3 (2) MFMA per
+// wave (the scale builtin with zero scales compiles to the unscaled instruction).
+template <int FMT>
+__global__ __launch_bounds__(512) void mfma_f8f6_16_k(float* __restrict__ sink, int iters, int seed) {
     v8i a, b;
 #pragma unroll
     for (int i = 0; i < 8; i++) {
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(512) void mfma_f8_16_k(float* __restrict__ sink, in
     for (int it = 0; it < iters; it++) {
 #pragma unroll
         for (int j = 0; j < 8; j++)
-            c[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4((j & 1) ? a : b, (j & 2) ? a : b, c[j], 0, 0,
+            c[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4((j & 1) ? a : b, (j & 2) ? a : b, c[j], FMT, FMT,
                                                                     0, 0, 0, 0);
     }
     float s = 0.f;
@@ -584,7 +586,14 @@ int rt4p_empty(int blocks, int threads, void* stream) {
 
 int rt4p_mfma_f8_16x16(void* sink, int iters, int blocks, void* stream) {
     if (!sink || iters < 1 || blocks < 1) return 1;
-    hipLaunchKernelGGL(mfma_f8_16_k, dim3(blocks), dim3(512), 0, (hipStream_t)stream, static_cast<float*>(sink),
+    hipLaunchKernelGGL(mfma_f8f6_16_k<0>, dim3(blocks), dim3(512), 0, (hipStream_t)stream, static_cast<float*>(sink),
+                       iters, 12345);
+    return last() == hipSuccess ? 0 : 3;
+}
+
+int rt4p_mfma_f6_16x16(void* sink, int iters, int blocks, void* stream) {
+    if (!sink || iters < 1 || blocks < 1) return 1;
+    hipLaunchKernelGGL(mfma_f8f6_16_k<2>, dim3(blocks), dim3(512), 0, (hipStream_t)stream, static_cast<float*>(sink),
                        iters, 12345);
     return last() == hipSuccess ? 0 : 3;
 }

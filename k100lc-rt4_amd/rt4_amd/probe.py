@@ -7,7 +7,8 @@ import pathlib
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent / "lib" / "librt4probe.so"
 EXPORTS = ("rt4p_hbm_read", "rt4p_read_burst", "rt4p_copy", "rt4p_mfma_i8", "rt4p_valu_fma", "rt4p_gemv_loads",
-           "rt4p_empty", "rt4p_mfma_f8f6f4", "rt4p_mfma_f8_16x16", "rt4p_gemm_unit")
+           "rt4p_empty", "rt4p_mfma_f8f6f4", "rt4p_mfma_f8_16x16", "rt4p_mfma_f6_16x16",
+           "rt4p_gemm_unit")
 _lib = None
 
 
@@ -24,7 +25,7 @@ def lib() -> ctypes.CDLL:
                 "rt4p_copy": [P, P, Z, I, P],
                 "rt4p_mfma_i8": [P, I, I, I, P], "rt4p_valu_fma": [P, I, I, P],
                 "rt4p_gemv_loads": [P, P, P, P, P, I, I, I, I, I, I, I, P], "rt4p_empty": [I, I, P],
-                "rt4p_mfma_f8f6f4": [P, I, I, I, P], "rt4p_mfma_f8_16x16": [P, I, I, P],
+                "rt4p_mfma_f8f6f4": [P, I, I, I, P], "rt4p_mfma_f8_16x16": [P, I, I, P], "rt4p_mfma_f6_16x16": [P, I, I, P],
                 "rt4p_gemm_unit": [P, I, I, I, P]}
         for name, args in sigs.items():
             getattr(L, name).argtypes = args
@@ -221,16 +222,21 @@ def launch_cost(torch, timed_graph, n: int = 64) -> float:
     return round(timed_graph(torch, fn) * 1e3 / n, 3)
 
 
-def mfma_f8_16x16_rate(torch, iters: int = 2048) -> float:
-    """Measured dense rate (TOPS) of v_mfma_f32_16x16x128_f8f6f4 with FP8 operands and
-    no block scale, as the attention kernel issues it: 2 waves per SIMD, 8
-    independent accumulator chains per wave."""
+def mfma_f8f6_16x16_rates(torch, iters: int = 2048) -> dict:
+    """Measured dense rate (TOPS) of v_mfma_f32_16x16x128_f8f6f4 without a block scale, as the
+    attention issues it (FP6 over its staged copy, FP8 in tiles a workgroup stages itself),
+    and its cycles per instruction and SIMD at 2.4 GHz: 2 waves per SIMD, 8 independent
+    accumulator chains per wave."""
     L = lib()
     cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
     sink = torch.zeros(1 << 16, dtype=torch.float32, device="cuda")
     st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    ms = _timed(torch, lambda: L.rt4p_mfma_f8_16x16(ctypes.c_void_p(sink.data_ptr()), iters, cus, st))
-    return round(2.0 * 32768 * 8 * iters * 8 * cus / ms / 1e9, 1)
+    out = {}
+    for fn, name in ((L.rt4p_mfma_f8_16x16, "fp8"), (L.rt4p_mfma_f6_16x16, "fp6")):
+        ms = _timed(torch, lambda: fn(ctypes.c_void_p(sink.data_ptr()), iters, cus, st))
+        out[f"mfma_f32_16x16x128_{name}_TOPS"] = round(2.0 * 32768 * 8 * iters * 8 * cus / ms / 1e9, 1)
+        out[f"mfma_f32_16x16x128_{name}_cycles"] = round(ms * 1e-3 * 2.4e9 / (8 * iters * 2), 1)
+    return out
 
 
 def mfma_f8f6f4_rates(torch, iters: int = 2048) -> dict:
