@@ -52,6 +52,7 @@ KERNELS = {                       # report key -> substring of the rocprof kerne
     "gemv_gate_up": "gemv_w4a8_tl_k<4",
     "gemv_c0": "gemv_w4a8_dot_k<2, 5",
     "gemm_gate_up": "gemm_w4a8_k<",
+    "gemm_gate_up_combine": "gemm_combine_k<",
     "attention_c4": "fa_int4_k",
     "attention_c4_staging": "fa_expand_kv_k",
 }
@@ -59,6 +60,7 @@ LABELS = {
     "gemv_gate_up": "gate/up GEMV (M=4, K=5120, N=17408)",
     "gemv_c0": "C0 GEMV (M=1, K=5120, N=5120)",
     "gemm_gate_up": "gate/up prefill GEMM (M=1024, K=5120, N=17408)",
+    "gemm_gate_up_combine": "gate/up prefill GEMM, sum of the split tiles (once per call)",
     "attention_c4": "C4 attention (1024 queries over 33792 keys, 24/4 heads, D=256)",
     "attention_c4_staging": "C4 attention K/V staging pass (once per call)",
 }
@@ -97,10 +99,24 @@ def attention_staging_bytes(n_kv: int, KVH: int, D: int = 256) -> int:
     return 2 * KVH * n_kv * D // 2 + 2 * KVH * n_tile * 12288
 
 
+def gemm_combine_bytes(M: int, N: int, K: int, cus: int = 256) -> int:
+    """The prefill GEMM's combining launch where every left-over 128 x 256 tile is cut into
+    cus / tiles pieces (M=1024, N=17408: 32 tiles in 8): each fp32 partial tile read once, the
+    tile written once."""
+    tiles = -(-M // 128) * -(-N // 256) % cus
+    pieces = min(cus // tiles, K // 128) if tiles else 0
+    return tiles * (pieces + 1) * 128 * 256 * 4
+
+
+# The kernels of one call: their traffic is also given as a sum, against the first one's
+# algorithmic bytes (the others move only what this implementation adds).
+PER_CALL = {"gemm_gate_up": ("gemm_gate_up", "gemm_gate_up_combine"),
+            "attention_c4": ("attention_c4", "attention_c4_staging")}
 ALGO_BYTES = {
     "gemv_gate_up": gemv_bytes(4, 17408, 5120),
     "gemv_c0": gemv_bytes(1, 5120, 5120),
     "gemm_gate_up": gemm_bytes(1024, 17408, 5120),
+    "gemm_gate_up_combine": gemm_combine_bytes(1024, 17408, 5120),
     "attention_c4": attention_bytes(1024, 32768 + 1024, 24, 4)["total"],
     "attention_c4_staging": attention_staging_bytes(32768 + 1024, 4),
 }
@@ -150,6 +166,11 @@ def summarize(fetch_csv: str, write_csv: str) -> dict:
             d["traffic_bytes"] = d["fetch_bytes"] + d["write_bytes"]
             d["algorithmic_bytes"] = ALGO_BYTES[key]
             d["traffic_over_algorithmic"] = round(d["traffic_bytes"] / ALGO_BYTES[key], 3)
+    for key, parts in PER_CALL.items():
+        if all("traffic_bytes" in res.get(p, {}) for p in parts):
+            n = sum(res[p]["traffic_bytes"] for p in parts)
+            res[key]["per_call_traffic_bytes"] = n
+            res[key]["per_call_over_algorithmic"] = round(n / ALGO_BYTES[key], 3)
     return res
 
 
@@ -178,6 +199,10 @@ def traffic_md(res: dict, fetch_csv: str, write_csv: str) -> str:
         out.append(f"| {LABELS[key]} `{KERNELS[key]}...` | {d['dispatches']} | {d['fetch_bytes']:,} | "
                    f"{d['write_bytes']:,} | {d['traffic_bytes']:,} | {d['algorithmic_bytes']:,} | "
                    f"{d['traffic_over_algorithmic']:.3f} |")
+        if "per_call_traffic_bytes" in d:
+            out.append(f"| {LABELS[key].split(' (')[0]}, whole call ({' + '.join(KERNELS[p] for p in PER_CALL[key])}) | "
+                       f"{d['dispatches']} | | | {d['per_call_traffic_bytes']:,} | {d['algorithmic_bytes']:,} | "
+                       f"{d['per_call_over_algorithmic']:.3f} |")
     ab = attention_bytes(1024, 32768 + 1024, 24, 4)
     out += ["", "Algorithmic bytes are each operand read once and each output written once "
             "(`rt4_amd.profiling.gemv_bytes`, `gemm_bytes`, `attention_bytes`); for the attention: " +

@@ -99,6 +99,24 @@ def test_traffic_and_sq_markdown_carry_the_json_numbers(tmp_path):
     assert "| VALU per MFMA | 10.0 |" in md
 
 
+def test_traffic_of_a_call_sums_its_kernels(tmp_path):
+    """The GEMM's combining launch is a key of its own and the call's traffic their sum."""
+    from rt4_amd import profiling
+    gemm = "void rt4::(anonymous namespace)::gemm_w4a8_k<4, false, false>(...)"
+    comb = "void rt4::(anonymous namespace)::gemm_combine_k<4>(...)"
+    copy = "void (anonymous namespace)::copy_k(uint4*, uint4 const*, unsigned long)"
+    kib = profiling.COPY_BYTES // 1024
+    _write_csv(tmp_path / "f.csv", [(copy, "FETCH_SIZE", kib), (gemm, "FETCH_SIZE", 1000.0), (comb, "FETCH_SIZE", 300.0)])
+    _write_csv(tmp_path / "w.csv", [(copy, "WRITE_SIZE", kib), (gemm, "WRITE_SIZE", 100.0), (comb, "WRITE_SIZE", 40.0)])
+    res = profiling.summarize(str(tmp_path / "f.csv"), str(tmp_path / "w.csv"))
+    assert res["gemm_gate_up"]["traffic_bytes"] == 1100 * 1024
+    assert res["gemm_gate_up_combine"]["traffic_bytes"] == 340 * 1024
+    assert res["gemm_gate_up"]["per_call_traffic_bytes"] == 1440 * 1024
+    assert f"{1440 * 1024:,}" in profiling.traffic_md(res, "f.csv", "w.csv")
+    # 544 tiles on 256 CUs: 32 left over in 8 pieces of 128 KB, and the 32 tiles written
+    assert profiling.gemm_combine_bytes(1024, 17408, 5120) == 32 * 9 * 131072
+
+
 def test_sq_summary_fractions(tmp_path):
     from rt4_amd import profiling
     gemm = "void rt4::(anonymous namespace)::gemm_w4a8_k<false>(...)"
