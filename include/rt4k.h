@@ -272,13 +272,13 @@ int rt4_attention_prefill(float* out, const uint32_t* qq, const float* qsc, cons
                           int off, int n_tile, int n_heads, int ratio, int kv_cap, void* stream);
 
 /* Same, with an explicit number of KV splits per (64-row query block, head)
- * (tuning and tests; 0 selects the default that balances the grid over the
- * device's CUs; at most 64).  With more than one split each split writes its
+ * (tuning and tests; 0 selects the default, see rt4_attention_launch_plan; at most
+ * 64).  With more than one split each split writes its
  * partial state (unnormalised output, running max, denominator) to library scratch
- * (grown with hipMalloc), and the partial states are combined in split order: by the
- * split that finishes last for a (query block, head) within the same launch (up to 4
- * splits of a large grid; one counter per (query block, head)), else by a launch of
- * their own. */
+ * (grown with hipMalloc), and the partial states are combined in a fixed order (the
+ * outputs in split order): by the split that finishes last for a (query block, head)
+ * within the same launch (up to 4 splits of a large grid; one counter per (query
+ * block, head)), else by a launch of their own. */
 int rt4_attention_prefill_cfg(float* out, const uint32_t* qq, const float* qsc, const uint32_t* kc,
                               const float* ksc, const uint32_t* vc, const float* vsc, int n_q, int n_kv,
                               int off, int n_tile, int n_heads, int ratio, int kv_cap, int kv_splits,
